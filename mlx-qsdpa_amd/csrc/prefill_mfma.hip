@@ -359,15 +359,31 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
   // XCD-aware work order: workgroups are dispatched to the 8 XCDs round
   // robin, so the work of workgroup id w goes to XCD w % 8 in consecutive
   // runs: the row groups of one (batch, kv head) share one XCD's L2.
+  //
+  // Causal calls of several rounds of workgroups: a row group's work grows
+  // with its position, so each head's groups run from the longest down (the
+  // last workgroups to start are then the shortest), and where the heads do
+  // not divide evenly over the XCDs the heads alternate instead, so that no
+  // XCD holds only long groups.  A prompt of 3000 tokens (32 / 8 heads,
+  // 4-bit; 752 workgroups), with its cache update: 142.6 us against 156.5
+  // with the shortest groups first.
   const int total = gridDim.x;
-  int w = blockIdx.x;
-  if (total % 8 == 0) w = (w % 8) * (total / 8) + w / 8;
+  const int heads = p.Hkv * p.B;
   const int S = p.num_splits;
-  const int split = w % S;
-  w /= S;
-  const int grp = w % groups_per_head;
-  const int kvh = (w / groups_per_head) % p.Hkv;
-  const int b = w / (groups_per_head * p.Hkv);
+  int w = blockIdx.x, split = 0, grp, head;
+  if (p.causal && S == 1 && heads % 8 != 0) {
+    head = w % heads;
+    grp = w / heads;
+  } else {
+    if (total % 8 == 0) w = (w % 8) * (total / 8) + w / 8;
+    split = w % S;
+    w /= S;
+    grp = w % groups_per_head;
+    head = w / groups_per_head;
+  }
+  if (p.causal) grp = groups_per_head - 1 - grp;
+  const int kvh = head % p.Hkv;
+  const int b = head / p.Hkv;
 
   const int rows = p.G * p.qL;
   const int v_first = grp * kPGroupRows;

@@ -113,6 +113,20 @@ def test_prefill_key_splits(device, case):
         _check(q, kq, vq, bits, gs, f"split case {case} kv_start", causal=True, kv_start=ks)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,L", [(1, 12, 3, 1500), (1, 16, 1, 2100), (1, 32, 8, 1100)])
+def test_prefill_causal_rounds(device, B, Hq, Hkv, L):
+    """Causal prompts of several rounds of workgroups, whose row groups run
+    from the longest down: heads that alternate over the XCDs (3 and 1) and
+    heads in runs (8), each with a partial last group.  Every row group is
+    computed exactly once."""
+    q, kq, vq = _inputs(B, Hq, Hkv, L, L, 4, 64, torch.float16, seed=L)
+    splits, _ = kernels.decode_plan(q, kq[0], vq[0], kq[1], vq[1], kq[2], vq[2], scale=128 ** -0.5, bits=4,
+                                    group_size=64)
+    assert splits == 1 and Hq // Hkv * L % 128 != 0
+    print(f"prefill causal rounds Hkv={Hkv} L={L}", flush=True)
+    _check(q, kq, vq, 4, 64, f"rounds Hkv={Hkv}", causal=True)
+
+
 @pytest.mark.parametrize("N", [1, 63, 64, 65, 130, 191])
 def test_prefill_short_key_ranges(device, N):
     """One to three 64-key tiles (full and partial): the pipeline dequantizes
