@@ -110,7 +110,7 @@ typedef struct {
   const int32_t* kv_start;
 
   /* 0 = choose automatically, 1 = single pass, >1 = split-K with this many
-   * splits per (batch, kv head).  With kv_start and B > 1 (D in {128, 256})
+   * splits per (batch, kv head).  With kv_start and B > 1 (matrix-core path)
    * the count is an average: the batch's keys per kv head are cut into
    * num_splits * B equal runs of tiles over the sequences laid end to end
    * (a run may cross sequences; a sequence with no keys gets none).       */
@@ -133,7 +133,7 @@ typedef struct {
   void* prof_end;
 
   /* Query positions per (batch, head); 0 or 1 = one (a decode step).
-   * q_len > 1 needs D in {128, 256} and the alignment of the matrix-core
+   * q_len > 1 needs the alignment of the matrix-core
    * path (else QSDPA_ERR_UNSUPPORTED); mlx_qsdpa's dispatch.py:68-83 sends
    * such calls through dequantize + attention instead.                    */
   int32_t q_len;

@@ -119,7 +119,7 @@ int validate_decode(const qsdpa_decode_args* a) {
   if (a->q_len < 0) return fail(QSDPA_ERR_INVALID, "q_len must be >= 0, got %d", a->q_len);
   if (a->q_len > 1 && !mfma_supports(a))
     return fail(QSDPA_ERR_UNSUPPORTED,
-                "q_len=%d needs the matrix-core path (D 128 or 256, aligned views); use dequantize + attention",
+                "q_len=%d needs the matrix-core path (D 64, 128 or 256, aligned views); use dequantize + attention",
                 a->q_len);
   if (a->mask.ptr) {
     const int md = a->mask_dtype;
@@ -285,9 +285,9 @@ int run_decode(const qsdpa_decode_args* args, int splits, void* workspace, hipSt
   else rc = launch_decode_valu(args, splits, part_acc, part_ml, s);
   if (rc) return rc;
   // The MFMA kernels store float16 inputs' partials as normalised float16
-  // rows (in the first half of the float32 area).
+  // rows (in the first half of the float32 area), float32 ones at D = 64.
   if (splits > 1 && !fused)
-    rc = launch_merge(args, splits, part_acc, part_ml, mfma && args->dtype == QSDPA_F16, units ? sched : nullptr,
+    rc = launch_merge(args, splits, part_acc, part_ml, mfma && args->dtype == QSDPA_F16 && args->D != 64, units ? sched : nullptr,
                       units + args->B, s);
   return rc;
 }

@@ -323,7 +323,7 @@ __device__ __forceinline__ void decode_segment(const MfmaParams& p, float* s_acc
 template <typename Tag, int D, int CHUNK>
 __device__ __forceinline__ void split_merge(const MfmaParams& p, int* s_flag, int b, int kvh, int hblk, int first,
                                             int count) {
-  constexpr bool kHalf = Tag::kId == QSDPA_F16;  // float16 normalised partial rows
+  constexpr bool kHalf = half_parts<Tag, D>();  // float16 normalised partial rows
   constexpr int kPer = 8, kRowT = D / kPer;
   constexpr uint32_t kPast = 0x80000000u;  // an offset past every descriptor: reads zero
   typedef uint32_t u2 __attribute__((ext_vector_type(2)));
@@ -404,7 +404,7 @@ __device__ __forceinline__ void split_merge(const MfmaParams& p, int* s_flag, in
       for (int e = 0; e < kPer; ++e) acc[e] = fmaf(xv[e], we, acc[e]);
     }
   }
-  store_out8<Tag>(p, b, hh, iq, d, acc, L);
+  store_out8<Tag, D>(p, b, hh, iq, d, acc, L);
 }
 
 // Zero output rows of the block's 16 query rows for every sequence of the
@@ -422,7 +422,7 @@ __device__ __forceinline__ void zero_empty_sequences(const MfmaParams& p, int kv
 #pragma unroll
   for (int e = 0; e < kPer; ++e) zero[e] = 0.0f;
   for (int b = 0; b < p.B; ++b)
-    if (seq_tiles(p.kv_start, b, p.N) == 0) store_out8<Tag>(p, b, hh, iq, d, zero, 0.0f);
+    if (seq_tiles(p.kv_start, b, p.N) == 0) store_out8<Tag, D>(p, b, hh, iq, d, zero, 0.0f);
 }
 
 // APPEND: the folded append (p.knew / p.vnew; its own instantiations, so the
@@ -502,9 +502,13 @@ using DecodeKernel = void (*)(MfmaParams);
 
 template <typename Tag, int D, int BITS, bool SK, bool MASK, bool FUSED, bool APPEND>
 DecodeKernel by_gs(int gs) {
-  return gs == 32 ? decode_mfma_kernel<Tag, D, BITS, 32, SK, MASK, FUSED, APPEND>
-       : gs == 64 ? decode_mfma_kernel<Tag, D, BITS, 64, SK, MASK, FUSED, APPEND>
-                  : decode_mfma_kernel<Tag, D, BITS, 128, SK, MASK, FUSED, APPEND>;
+  if constexpr (D == 64)
+    return gs == 32 ? decode_mfma_kernel<Tag, D, BITS, 32, SK, MASK, FUSED, APPEND>
+                    : decode_mfma_kernel<Tag, D, BITS, 64, SK, MASK, FUSED, APPEND>;
+  else
+    return gs == 32 ? decode_mfma_kernel<Tag, D, BITS, 32, SK, MASK, FUSED, APPEND>
+         : gs == 64 ? decode_mfma_kernel<Tag, D, BITS, 64, SK, MASK, FUSED, APPEND>
+                    : decode_mfma_kernel<Tag, D, BITS, 128, SK, MASK, FUSED, APPEND>;
 }
 
 // The instantiation for a launch; null where none is built (the launcher
@@ -557,17 +561,24 @@ void launch_bits(const MfmaParams& p, int bits, int gs, hipStream_t stream, cons
 
 }  // namespace
 
-// The MFMA path covers D in {128, 256} for any GQA factor (heads padded to
+// D = 64 against the VALU kernel (decode_valu.hip), which takes only its
+// unaligned views now, wall us per call: B = 8, 32 / 8 heads over 8192 keys,
+// 4-bit f16 16.6 against 35.4, 8-bit bf16 19.2 against 42.2; B = 1 over 4096 /
+// 32768 keys 9.8 / 13.2 against 14.4 / 24.1; 16 left-padded sequences of
+// 2192 to 8192 keys (stream-K) 29.0 against 61.6.  It is VALU-bound: a tile
+// holds half the bytes of a D = 128 one under the same softmax.
+//
+// The MFMA path covers D in {64, 128, 256} for any GQA factor (heads padded to
 // blocks of 16).  Its vector loads need: q rows 4-byte aligned; K / V rows
 // aligned to the per-lane piece (16 B for the K quarter when it is >= 16 B,
 // the V piece size otherwise); scale / bias rows 4-byte aligned when a K
 // quarter spans two groups (D = 256, group_size = 32).
 bool mfma_supports(const qsdpa_decode_args* a) {
-  if (a->D != 128 && a->D != 256) return false;
+  if (a->D != 64 && a->D != 128 && a->D != 256) return false;
   if (a->group_size != 32 && a->group_size != 64 && a->group_size != 128) return false;
   if (!aligned_view(a->q, 4, 2)) return false;
   const int kq_bytes = a->D / 4 * a->bits / 8;             // K quarter row
-  const int vp_bytes = a->D / 16 * a->bits / 8;            // V piece per token
+  const int vp_bytes = std::max(a->D / 16 * a->bits / 8, 4);  // V piece per token (at least a word)
   if (!aligned_view(a->k_packed, std::min(kq_bytes, 16), 4)) return false;
   if (!aligned_view(a->v_packed, std::min(vp_bytes, 16), 4)) return false;
   if (a->D / 4 / a->group_size == 2) {
@@ -633,7 +644,10 @@ int launch_decode_mfma(const qsdpa_decode_args* a, int num_splits, float* part_a
   if (append && (a->D != 128 || a->mask.ptr))
     return fail(QSDPA_ERR_UNSUPPORTED, "decode_mfma: the folded append is built for D=128 without a mask");
   const bool f16 = a->dtype == QSDPA_F16;
-  if (a->D == 128) {
+  if (a->D == 64) {
+    if (f16) launch_bits<F16, 64>(p, a->bits, a->group_size, stream, a);
+    else launch_bits<BF16, 64>(p, a->bits, a->group_size, stream, a);
+  } else if (a->D == 128) {
     if (f16) launch_bits<F16, 128>(p, a->bits, a->group_size, stream, a);
     else launch_bits<BF16, 128>(p, a->bits, a->group_size, stream, a);
   } else {

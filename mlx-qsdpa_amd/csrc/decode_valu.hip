@@ -1,5 +1,5 @@
-// Split-K quantized decode on the VALU (any GQA factor; the MFMA kernel in
-// decode_mfma.hip takes over for head groups of 16).
+// Split-K quantized decode on the VALU, for views whose alignment the MFMA
+// kernel in decode_mfma.hip does not take.
 //
 // Reference: the single-pass kernel mlx_qsdpa/kernels.py:42-160 and the
 // split-K pass 1 / pass 2 kernels kernels.py:224-318 / 342-418.

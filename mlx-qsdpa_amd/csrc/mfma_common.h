@@ -22,6 +22,13 @@ typedef __bf16 b8 __attribute__((ext_vector_type(8)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u4 __attribute__((ext_vector_type(4)));
 
+// Whether split partials are normalised rows in float16: float16 inputs,
+// except at D = 64, where they stay float32.
+template <typename Tag, int D>
+constexpr bool half_parts() {
+  return Tag::kId == QSDPA_F16 && D != 64;
+}
+
 struct MfmaParams {
   int B, Hq, Hkv, N, G, hb_count, num_splits;
   float qscale;  // softmax scale * log2(e)

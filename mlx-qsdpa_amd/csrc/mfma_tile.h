@@ -29,7 +29,14 @@ struct Geo {
   static constexpr int KW = QD * BITS / 32;     // K words per lane per half
   static constexpr int WPS = BITS / 4;          // words per 8-dim slice
   static constexpr int KG = QD >= GS ? QD / GS : 1;  // groups per K quarter (1 or 2)
-  static constexpr int VW = NB * BITS / 32;     // V words per lane per token
+  // D = 64 with 4-bit codes: a lane's V piece (4 dims) is half a word, so
+  // lanes 2i and 2i + 1 load one word and each takes its half.
+  static constexpr bool HalfV = NB * BITS < 32;
+  static constexpr int VW = HalfV ? 1 : NB * BITS / 32;  // V words per lane per token
+  // D = 64: P enters P.V as two 16-bit terms for float16 too, and split
+  // partials stay float32 (the kernel that these calls took before, and the
+  // dequantize + attention path of several positions, keep both in 32 bits).
+  static constexpr bool Wide = D == 64;
   static constexpr int RW = D * BITS / 32;      // words per row
   static constexpr int NG = D / GS;             // groups (scales) per row
   static constexpr int ND = NG >= 2 ? NG / 2 : 1;  // 32-bit meta words per row
@@ -102,6 +109,7 @@ struct VMetaLane {
   int src[4];
   uint32_t sel;
   uint32_t shift;
+  uint32_t vsel;  // HalfV: the v_perm_b32 selector of the lane's half of two V words
 };
 
 // Buffer descriptors over rows [s0, s0 + len) of (batch b, kv head kvh) of
@@ -146,7 +154,7 @@ __device__ __forceinline__ void lane_setup(const Rsrcs& rs, int quad, int r, Lan
   L.k_r = PK ? quad * G::KW * 4 + (r >> 3) * 16 + (r & 7) * rs.k_sn : quad * G::KW * 4 + r * rs.k_sn;
   L.ks_r = kg0 * 2 + r * rs.ks_sn;
   L.kb_r = kg0 * 2 + r * rs.kb_sn;
-  L.v_r = r * G::VW * 4 + 4 * quad * rs.v_sn;
+  L.v_r = (G::HalfV ? r / 2 : r * G::VW) * 4 + 4 * quad * rs.v_sn;
   L.vs_r = vword * 4 + r * rs.vs_sn;
   L.vb_r = vword * 4 + r * rs.vb_sn;
   // Opaque to the optimizer: seeing r * stride inside, it folds a load's
@@ -161,6 +169,7 @@ __device__ __forceinline__ void lane_setup(const Rsrcs& rs, int quad, int r, Lan
   for (int k = 0; k < 4; ++k) vm.src[k] = (16 * dw + 4 * quad + k) * 4;
   vm.sel = half ? 0x07060302u : 0x05040100u;
   vm.shift = half ? 0u : 16u;
+  vm.vsel = (r & 1) ? 0x07060302u : 0x05040100u;
 }
 
 template <typename Tag, int D, int BITS, int GS>
@@ -274,8 +283,23 @@ struct Kernel {
   // sv2 / bv2: V scale / bias pairs of tokens (2i, 2i+1) of the lane's group.
   template <typename IV>
   static __device__ __forceinline__ void pv_f16(Regs& R, const uint32_t (&sv2)[4], const uint32_t (&bv2)[4],
-                                                const uint32_t (&pb)[4], f4 (&acc)[G::NB], IV&& issue_v) {
-    if constexpr (BITS == 4) {
+                                                const uint32_t (&pb)[4], const uint32_t (&pb_lo)[4], uint32_t vsel,
+                                                f4 (&acc)[G::NB], IV&& issue_v) {
+    if constexpr (G::HalfV) {
+      // X: the lane's 4 nibbles of tokens (2i, 2i+1).
+      uint32_t X[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) X[i] = perm(R.vw[2 * i + 1][0], R.vw[2 * i][0], vsel);
+      issue_v(R);
+#pragma unroll
+      for (int nb = 0; nb < G::NB; ++nb) {
+        uint32_t a[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[i] = f16x2_fma(nib_codes(X[i], X[i] >> 8, nb), sv2[i], bv2[i]);
+        acc[nb] = mfma<Tag>(a, pb, acc[nb]);
+        acc[nb] = mfma<Tag>(a, pb_lo, acc[nb]);
+      }
+    } else if constexpr (BITS == 4) {
       // X: nibbles 0-3 of tokens (2i, 2i+1), Y: nibbles 4-7.
       uint32_t X[4][G::VW], Y[4][G::VW];
 #pragma unroll
@@ -318,6 +342,7 @@ struct Kernel {
           a[i] = f16x2_fma(f16x2_sub1024(t), sv2[i], bv2[i]);
         }
         acc[nb] = mfma<Tag>(a, pb, acc[nb]);
+        if constexpr (G::Wide) acc[nb] = mfma<Tag>(a, pb_lo, acc[nb]);
       }
     }
   }
@@ -360,7 +385,12 @@ struct Kernel {
     }
     if constexpr (MASK) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) sc[j] += mv[j];
+      for (int j = 0; j < 8; ++j) {
+        // (D = 64 masks as the dequantize + attention path does: the score of
+        // a masked key is replaced, whatever it was.)
+        if constexpr (G::Wide) sc[j] = mv[j] == -__builtin_huge_valf() ? mv[j] : sc[j] + mv[j];
+        else sc[j] += mv[j];
+      }
     }
     if (__builtin_expect(tb + kTile > n1 || tb < n0, 0)) {  // a partial tile
 #pragma unroll
@@ -388,7 +418,7 @@ struct Kernel {
     uint32_t pb[4], pb_lo[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i) pb[i] = pack_T2<Tag>(pr[2 * i], pr[2 * i + 1]);
-    if constexpr (Tag::kId == QSDPA_BF16) {
+    if constexpr (Tag::kId == QSDPA_BF16 || G::Wide) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
         pb_lo[i] = pack_T2<Tag>(pr[2 * i] - unpack_T2_lo<Tag>(pb[i]),
@@ -411,7 +441,7 @@ struct Kernel {
         sv2[i] = perm(dS[2 * i + 1], dS[2 * i], vm.sel);
         bv2[i] = perm(dB[2 * i + 1], dB[2 * i], vm.sel);
       }
-      pv_f16(R, sv2, bv2, pb, acc, issue_v);
+      pv_f16(R, sv2, bv2, pb, pb_lo, vm.vsel, acc, issue_v);
     } else {
       float svf[8], bvf[8];
 #pragma unroll
@@ -425,8 +455,10 @@ struct Kernel {
         for (int j = 0; j < 8; ++j)
 #pragma unroll
           for (int w = 0; w < G::VW; ++w) {
-            lo[j][w] = R.vw[j][w] & 0x0F0F0F0Fu;         // nibbles 0, 2, 4, 6 as bytes
-            hi[j][w] = (R.vw[j][w] >> 4) & 0x0F0F0F0Fu;  // nibbles 1, 3, 5, 7
+            // (HalfV: the lane's half of the word at the bottom.)
+            const uint32_t x = G::HalfV ? perm(0u, R.vw[j][w], vm.vsel) : R.vw[j][w];
+            lo[j][w] = x & 0x0F0F0F0Fu;         // nibbles 0, 2, 4, 6 as bytes
+            hi[j][w] = (x >> 4) & 0x0F0F0F0Fu;  // nibbles 1, 3, 5, 7
           }
       }
 #pragma unroll
@@ -719,15 +751,19 @@ struct Kernel {
 constexpr int kCoherent = 16;
 
 // A normalised output row piece: out[b, hh, iq, d .. d + 8) = v / L (0 when
-// L = 0: every key of the row was masked or absent).  Output rows are only
+// L = 0: every key of the row was masked or absent; D = 64: also when L is
+// NaN, as the path these calls took before).  Output rows are only
 // 2-byte aligned in general: stores of 16-bit halves.
-template <typename Tag>
+template <typename Tag, int D>
 __device__ __forceinline__ void store_out8(const MfmaParams& p, int b, int hh, int iq, int d, const float (&v)[8],
                                            float L) {
   const float inv = L > 0.0f ? 1.0f / L : 0.0f;
   uint32_t pk[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) pk[e] = pack_T2<Tag>(v[2 * e] * inv, v[2 * e + 1] * inv);
+  if constexpr (D == 64) {
+    if (!(L > 0.0f)) pk[0] = pk[1] = pk[2] = pk[3] = 0u;
+  }
   uint16_t* dst = p.out + static_cast<int64_t>(b) * p.o_sb + static_cast<int64_t>(hh) * p.o_sh +
                   static_cast<int64_t>(iq) * p.o_sq + d;
 #pragma unroll
@@ -747,7 +783,7 @@ __device__ __forceinline__ void store_out8(const MfmaParams& p, int b, int hh, i
 // kvh * G + v % G) and column x: local(v) + x.
 template <typename Tag, int D>
 struct PartRows {
-  static constexpr int kEsz = Tag::kId == QSDPA_F16 ? 2 : 4;  // float16 normalised rows, or float32 sums
+  static constexpr int kEsz = half_parts<Tag, D>() ? 2 : 4;  // float16 normalised rows, or float32 sums
   rsrc_t acc, ml;
   int64_t first;
   __device__ __forceinline__ PartRows(const MfmaParams& p, int b, int kvh) {
@@ -804,18 +840,27 @@ __device__ __forceinline__ void merge_store(const MfmaParams& p, RowF&& row_of, 
       v[4] = fmaf(a1[0], f, v[4]); v[5] = fmaf(a1[1], f, v[5]);
       v[6] = fmaf(a1[2], f, v[6]); v[7] = fmaf(a1[3], f, v[7]);
     }
+    if constexpr (D == 64) {
+      // A NaN sum makes the whole row zero (store_out8); its partial must not
+      // spread NaN beyond that.
+      if (!(L > 0.0f)) {
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) v[e] = 0.0f;
+        if (L != 0.0f) Mh = 0.0f;
+      }
+    }
     const int vh = v0 + h;
     const int hh = kvh * p.G + vh % p.G;  // head and query position of the row
     const int iq = vh / p.G;
     if (p.num_splits == 1 || (FUSED && direct)) {
-      store_out8<Tag>(p, b, hh, iq, d, v, L);
+      store_out8<Tag, D>(p, b, hh, iq, d, v, L);
     } else if (FUSED) {
       // Partials merged inside this launch (split_merge): agent-coherent
       // stores through the block's descriptors.
       if constexpr (FUSED) {
       const PartRows<Tag, D> pr(p, b, kvh);
       const uint32_t slot = PartRows<Tag, D>::local(p, vh) + col;
-      if constexpr (Tag::kId == QSDPA_F16) {
+      if constexpr (half_parts<Tag, D>()) {
         const float inv = L > 0.0f ? 1.0f / L : 0.0f;
         const u4 w = u4{pack_T2<Tag>(v[0] * inv, v[1] * inv), pack_T2<Tag>(v[2] * inv, v[3] * inv),
                         pack_T2<Tag>(v[4] * inv, v[5] * inv), pack_T2<Tag>(v[6] * inv, v[7] * inv)};
@@ -839,7 +884,7 @@ __device__ __forceinline__ void merge_store(const MfmaParams& p, RowF&& row_of, 
       const int64_t prow = static_cast<int64_t>(hh) * p.qL + iq;
       const int64_t slot = p.units ? prow * (p.units + p.B) + col
                                    : (static_cast<int64_t>(b) * p.Hq * p.qL + prow) * p.num_splits + col;
-      if constexpr (Tag::kId == QSDPA_F16) {
+      if constexpr (half_parts<Tag, D>()) {
         // float16 rows of the split's normalised output (acc / L, within
         // the range of V), so the partials are half the bytes.  Plain
         // stores: with the K / V stream non-temporal the rows stay in the

@@ -15,9 +15,9 @@ choices:
 * Several query positions (qL > 1: speculative or chunked decoding,
   prefill) run on the fused matrix-core kernel, including mask="causal"
   (aligned to the last key), where the reference dequantizes and runs SDPA.
-  Shapes that kernel does not take (D = 64, unaligned views) keep the
-  reference's path: HIP dequantize, then float32 attention with torch on
-  the GPU (dispatch.py:68-83).
+  Shapes that kernel does not take (unaligned views; at D = 64 short key
+  ranges and additive masks) keep the reference's path: HIP dequantize, then
+  float32 attention with torch on the GPU (dispatch.py:68-83).
 
 Head dims the library does not compile (any other multiple of 32, e.g. 32
 or 512, which the reference's validation accepts: dispatch.py:48-49) take
@@ -165,8 +165,10 @@ def quantized_sdpa(
     if isinstance(kv_start, torch.Tensor) and q.device.type == "cuda":
         kv_start = kernels.to_device(kv_start, q.device)
 
-    if D not in kernels.HEAD_DIMS or (qL > 1 and not _fused_takes(
-            q, packed_k, packed_v, k_scales, v_scales, k_biases, v_biases, scale, bits, group_size)):
+    if D not in kernels.HEAD_DIMS or (qL > 1 and not (
+            (D != 64 or _d64_in_kernel(mask, kv_start, B, H_q, qL, N))
+            and _fused_takes(q, packed_k, packed_v, k_scales, v_scales, k_biases, v_biases, scale, bits,
+                             group_size))):
         return fallback_sdpa(q, (packed_k, k_scales, k_biases),    # dispatch.py:68-83
                              (packed_v, v_scales, v_biases), bits=bits, group_size=group_size,
                              scale=scale, mask=mask, kv_start=kv_start)
@@ -203,10 +205,36 @@ def _row_aligned(t):
     return t.contiguous()
 
 
+# At D = 64 several query positions take the fused kernel from this many keys
+# on (a causal prompt of 1500 tokens, 32 / 8 heads: 114 us against 878 on the
+# dequantize + attention path); shorter calls are bound by their launches
+# either way.
+D64_FUSED_KEYS = 256
+
+
+def _d64_in_kernel(mask, kv_start, B, H_q, qL, N):
+    """Whether several positions at D = 64 run fused: enough keys, and masked
+    as the dequantize + attention path masks them ("causal" or a bool mask
+    over all keys, one start per sequence).  The path's other masks stay on
+    it: additive ones (a row whose every score is the type's lowest value
+    averages V there and is empty in the kernel, which scales the mask to
+    base 2), masks that broadcast over the keys."""
+    if N < D64_FUSED_KEYS:
+        return False
+    if kv_start is not None and tuple(kv_start.shape) != (B,):
+        return False
+    if not isinstance(mask, torch.Tensor):
+        return True
+    if mask.dtype != torch.bool or not 1 <= mask.dim() <= 4:
+        return False
+    shape = (1,) * (4 - mask.dim()) + tuple(mask.shape)
+    return shape[3] == N and shape[2] in (1, qL) and shape[1] in (1, H_q) and shape[0] in (1, B)
+
+
 def _fused_takes(q, packed_k, packed_v, k_scales, v_scales, k_biases, v_biases, scale, bits,
                  group_size):
     """Whether the fused kernel takes several query positions for these
-    inputs (the matrix-core path: D 128 or 256, aligned views).  Extension:
+    inputs (the matrix-core path: D 64, 128 or 256, aligned views).  Extension:
     the reference sends every qL > 1 call to dequantize + attention."""
     if k_biases is None or v_biases is None:
         k_biases = v_biases = None
