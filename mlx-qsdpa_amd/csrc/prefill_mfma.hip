@@ -6,10 +6,10 @@
 // decode kernel (decode_mfma.hip) takes such calls in blocks of 16 query rows,
 // each of which loads and dequantizes the kv head's whole K / V again.  Here
 // one workgroup takes 128 rows of a kv head -- 8 waves x 16 rows -- and every
-// K / V tile (64 tokens at D = 128, 32 at D = 256: the same number of
-// values) is loaded once per workgroup, dequantized once into LDS, and read
+// K / V tile (64 tokens at D = 128, 32 at D = 256, 128 at D = 64: the same
+// number of values) is loaded once per workgroup, dequantized once into LDS, and read
 // from LDS by all eight waves.  Per tile j, in each wave (described for
-// D = 128; PGeo gives the D = 256 shapes):
+// D = 128; PGeo gives the other shapes):
 //
 //   QK         S^T = K Q^T (A = K rows from LDS buffer j % 4, B = Q^T in
 //              registers): 4 token blocks x D/32 steps of v_mfma_f32_16x16x32
@@ -91,9 +91,16 @@ constexpr float kVBound = 64000.0f;          // largest |V| staged in float16 un
 // max|V| in the random tests), so one term keeps 2e-3 for |V| <= 8.
 constexpr float kPVSingle = 8.0f;
 
-// Tile geometry.  D = 128: 64-token tiles; D = 256: 32-token tiles, so that
-// a tile holds the same number of K / V values (and the four LDS buffers
-// still fit): the same MFMA, dequantization and LDS work per tile.
+// Tile geometry.  D = 128: 64-token tiles; D = 256: 32-token tiles and D =
+// 64: 128-token tiles, so that a tile holds the same number of K / V values
+// (and the four LDS buffers still fit): the same dequantization and LDS work
+// per tile, the same MFMA work too but for D = 64's second P term.
+//
+// D = 64 keeps what the dequantize + float32 attention path of these calls
+// held in 32 bits: P always enters P.V as two float16 terms (22 bits), split
+// partials are float32, a bfloat16 V is scaled to the top of float16's range
+// whatever its magnitude, and a row whose sum is NaN is zero.  Softmax bound:
+// twice the exponentials per MFMA of D = 128.
 //
 // LDS rows are padded.  Measured at the C5 chunk (D = 128): with 16-byte
 // padding (K 272 B, V^T 144 B per row) the 16-byte operand reads of the 16
@@ -105,7 +112,7 @@ constexpr float kPVSingle = 8.0f;
 // which is what fits four buffers in the LDS.
 template <int D>
 struct PGeo {
-  static constexpr int Tile = D == 256 ? 32 : 64;  // tokens per tile
+  static constexpr int Tile = D == 256 ? 32 : D == 128 ? 64 : 128;  // tokens per tile
   static constexpr int KPitch = D * 2 + 32;        // bytes per K row (token) in LDS
   static constexpr int VPitch = Tile * 2 + (D == 256 ? 16 : 32);  // bytes per V^T row (dim)
   static constexpr int KBytes = Tile * KPitch;
@@ -530,7 +537,10 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
       for (int e = 0; e < NE; ++e) sc[e] *= p.qscale;
       if constexpr (MASK) {
 #pragma unroll
-        for (int e = 0; e < NE; ++e) sc[e] += mv[e];
+        for (int e = 0; e < NE; ++e) {
+          if constexpr (D == 64) sc[e] = mv[e] == -__builtin_huge_valf() ? mv[e] : sc[e] + mv[e];
+          else sc[e] += mv[e];
+        }
       }
     }
     if (tb + kTile > n_wave) {  // keys past a row's limit (causal, or the sequence's end)
@@ -561,7 +571,8 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
     float s4[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) s4[t] = (pr[4 * t] + pr[4 * t + 1]) + (pr[4 * t + 2] + pr[4 * t + 3]);
-    if constexpr (NT == 4) lrun += (s4[0] + s4[1]) + (s4[2] + s4[3]);
+    if constexpr (NT == 8) lrun += ((s4[0] + s4[1]) + (s4[2] + s4[3])) + ((s4[4] + s4[5]) + (s4[6] + s4[7]));
+    else if constexpr (NT == 4) lrun += (s4[0] + s4[1]) + (s4[2] + s4[3]);
     else lrun += s4[0] + s4[1];
     // P^T of half u: k slots 2i, 2i + 1 = tokens tau(quad, 2i), tau(quad, 2i + 1):
     // blocks 2u (i = 0, 1) and 2u + 1 (i = 2, 3).
@@ -608,7 +619,7 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
   // to two tiles. ----
   typename P::Raw R0, R1;
   auto buf = [&](int j) { return s_buf + (j & 3) * PG::BufBytes; };
-  const int oob = len + 2 * kTile;  // rows past every descriptor: the loads read zero
+  const int oob = p.N - s0 + 2 * kTile;  // rows past every descriptor: the loads read zero
   auto row_of = [&](int j) { return j < T ? (j_base + j) * kTile : oob; };
   // Keys of tile j; past the split's tiles, the sequence end (every score
   // masked: an odd tile count's last pair computes one empty tile).
@@ -627,14 +638,16 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
     bool two = false;
     if constexpr (Tag::kId == QSDPA_BF16) {
       // max |V| of this workgroup's keys: a group's values are affine in
-      // the code, so its largest magnitude is at code 0 or 2^bits - 1.
+      // the code, so its largest magnitude is at code 0 or 2^bits - 1.  To
+      // the end of the last tile: keys past the causal limit are staged with
+      // it, and P = 0 does not cancel one that float16 cannot hold.
       constexpr int NG = D / GS;
       constexpr float kCodeMax = static_cast<float>((1 << BITS) - 1);
       // Eight rows per thread in flight (rows past the range read the
       // range's first row again: no effect on the maximum).
       constexpr int kRows = 8;
       float bound = 0.0f;
-      const int t_lo = j_base * kTile, t_hi = min((j_base + T) * kTile, len);
+      const int t_lo = j_base * kTile, t_hi = min((j_base + T) * kTile, p.N - s0);
       for (int t0 = t_lo + tid; t0 < t_hi; t0 += kRows * kPThreads) {
         uint16_t sv[kRows][NG], bv[kRows][NG];
 #pragma unroll
@@ -661,12 +674,13 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
 #pragma unroll
       for (int i = 0; i < kPWaves; ++i) bound = fmaxf(bound, s_red[i]);
       two = !(bound <= kPVSingle);
-      if (bound > kVBound) {
+      if (bound > kVBound || D == 64) {
         // k = 1 + floor(log2(bound / kVBound)), so that bound 2^-k < kVBound.
         // A finite bfloat16 bound (< 2^128) needs k <= 113; the clamp keeps
         // k <= 126 when the scan overflowed to Inf, so that 2^-k and 2^k
-        // stay normal floats.
-        const float x = fminf(bound * (1.0f / kVBound), 0x1p125f);
+        // stay normal floats.  D = 64: also up (k < 0), at least to k = -100,
+        // where 2^-k 2^24 is still finite.
+        const float x = fminf(D == 64 ? fmaxf(bound * (1.0f / kVBound), 0x1p-101f) : bound * (1.0f / kVBound), 0x1p125f);
         const int k = static_cast<int>((__builtin_bit_cast(uint32_t, x) >> 23) & 0xFFu) - 126;
         vsc = __builtin_bit_cast(float, static_cast<uint32_t>(127 - k) << 23);
         osc = __builtin_bit_cast(float, static_cast<uint32_t>(127 + k) << 23);
@@ -677,7 +691,9 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
     P::stage(R1, buf(1), tid, vsc);
     P::load(R1, src, row_of(3));
     __syncthreads();
-    if constexpr (Tag::kId == QSDPA_BF16) {
+    if constexpr (D == 64) {
+      run(std::true_type{});
+    } else if constexpr (Tag::kId == QSDPA_BF16) {
       if (two) run(std::true_type{});
       else run(std::false_type{});
     } else {
@@ -695,6 +711,12 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
   const int hq = kvh * p.G + v % p.G, iq = v / p.G;
   if (S == 1) {
     const float inv = (l > 0.0f ? 1.0f / l : 0.0f) * osc;
+    if constexpr (D == 64) {
+      if (!(l > 0.0f)) {
+#pragma unroll
+        for (int db = 0; db < PG::NB; ++db) acc[db] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+      }
+    }
     uint16_t* dst = p.out + static_cast<int64_t>(b) * p.o_sb + static_cast<int64_t>(hq) * p.o_sh +
                     static_cast<int64_t>(iq) * p.o_sq + 4 * quad;
 #pragma unroll
@@ -710,17 +732,26 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
   } else {
     // The split's partial of row (b, hq, iq), column `split`, then (m, l):
     // float16 inputs store the normalised row acc / l as float16 (as the
-    // decode kernel does); bfloat16 inputs store it as float32, with
+    // decode kernel does); bfloat16 inputs (and D = 64) store it as float32, with
     // (m + log2 l, 1) -- the same partial to the merge, whose weight for it
     // is l 2^(m - M) either way, but a sum that stays below max |V| where
     // acc itself would overflow float32 (rows of V near the bfloat16
     // maximum).
     const int64_t slot = ((static_cast<int64_t>(b) * p.Hq + hq) * p.qL + iq) * S + split;
     const float inv = l > 0.0f ? 1.0f / l : 0.0f;
+    if constexpr (D == 64) {
+      // A NaN sum makes the row zero in the merge, if nothing else of this
+      // partial is NaN.
+      if (!(l > 0.0f)) {
+#pragma unroll
+        for (int db = 0; db < PG::NB; ++db) acc[db] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+        if (l != 0.0f) mrun = 0.0f;
+      }
+    }
 #pragma unroll
     for (int db = 0; db < PG::NB; ++db) {
       const int d = 16 * db + 4 * quad;
-      if constexpr (Tag::kId == QSDPA_F16) {
+      if constexpr (half_parts<Tag, D>()) {
         typedef uint32_t u2 __attribute__((ext_vector_type(2)));
         *reinterpret_cast<u2*>(reinterpret_cast<uint16_t*>(p.part_acc) + slot * D + d) =
             u2{pack_T2<Tag>(acc[db][0] * inv, acc[db][1] * inv), pack_T2<Tag>(acc[db][2] * inv, acc[db][3] * inv)};
@@ -729,7 +760,7 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
       }
     }
     if (quad == 0) {
-      const bool norm = Tag::kId != QSDPA_F16 && l > 0.0f;
+      const bool norm = !half_parts<Tag, D>() && l > 0.0f;
       p.part_ml[slot * 2] = norm ? mrun + __log2f(l) : mrun;
       p.part_ml[slot * 2 + 1] = norm ? 1.0f : l;
     }
@@ -740,8 +771,10 @@ template <typename Tag, int D, int BITS, bool MASK>
 void launch_prefill_mask(const MfmaParams& p, int gs, int groups, hipStream_t stream, const qsdpa_decode_args* a) {
   const dim3 grid(groups * p.Hkv * p.B * p.num_splits);
   void (*k)(MfmaParams, int) = gs == 32 ? prefill_mfma_kernel<Tag, D, BITS, 32, MASK>
-                               : gs == 64 ? prefill_mfma_kernel<Tag, D, BITS, 64, MASK>
-                                          : prefill_mfma_kernel<Tag, D, BITS, 128, MASK>;
+                                        : prefill_mfma_kernel<Tag, D, BITS, 64, MASK>;
+  if constexpr (D != 64) {
+    if (gs == 128) k = prefill_mfma_kernel<Tag, D, BITS, 128, MASK>;
+  }
   if (a->prof_begin || a->prof_end)
     hipExtLaunchKernelGGL(k, grid, dim3(kPThreads), 0, stream, static_cast<hipEvent_t>(a->prof_begin),
                           static_cast<hipEvent_t>(a->prof_end), 0, p, groups);
@@ -760,16 +793,16 @@ void launch_prefill_gs(const MfmaParams& p, int gs, int groups, hipStream_t stre
 bool mfma_supports(const qsdpa_decode_args* a);
 
 // Tokens per tile (PGeo<D>::Tile) on the host.
-static int prefill_tile(int D) { return D == 256 ? PGeo<256>::Tile : PGeo<128>::Tile; }
+static int prefill_tile(int D) { return D == 256 ? PGeo<256>::Tile : D == 128 ? PGeo<128>::Tile : PGeo<64>::Tile; }
 
 // The prefill kernel takes q_len > 1 calls on the MFMA path's layouts whose
-// kv heads have at least one full 128-row group (D = 128 or 256); others stay
+// kv heads have at least one full 128-row group; others stay
 // on the decode kernel's 16-row blocks (a half-empty group would leave half
 // its waves computing padding rows).  K / V rows are read in 16-byte pieces
 // (8-byte V pieces at 4-bit), so the packed views must be aligned to the
 // pieces.  A thread's K piece (16 dims) always lies in one quantization group.
 bool prefill_supports(const qsdpa_decode_args* a) {
-  if (a->q_len <= 1 || (a->D != 128 && a->D != 256) || !mfma_supports(a)) return false;
+  if (a->q_len <= 1 || !mfma_supports(a)) return false;
   const int64_t rows = static_cast<int64_t>(a->H_q / a->H_kv) * a->q_len;
   if (rows < kPGroupRows) return false;
   // D = 256 only for calls with at least 2^24 (query row, key) pairs; below
@@ -785,6 +818,15 @@ bool prefill_supports(const qsdpa_decode_args* a) {
   // heads at q_len = 4 over 128K 58-59 against 73-75 us.
   if (a->D == 256 && static_cast<int64_t>(a->B) * a->H_q * a->q_len * a->N < (int64_t(1) << 24))
     return false;
+  // D = 64 from 5 * 2^20 pairs on.  Wall us per call, the decode kernel
+  // against this one: one sequence of 32 / 8 heads, q_len = 33 over 4096 /
+  // 8192 / 16384 keys 15.6 / 21.6 / 35.0 against 16.2 / 20.3 / 27.6 (4.3 /
+  // 8.7 / 17 million pairs), q_len = 100 over 1024 (3.3 million) 10.5 against
+  // 14.3, q_len = 300 over 600 (5.8 million) 19.9 against 19.2, 200 over 2048
+  // (13 million) 26.5 against 19.2; 8 / 2 heads, q_len = 100 over 4096 (3.3
+  // million) 13.1 against 15.7.  Prompts of 1500 / 3000 tokens 98.6 / 252
+  // against 36.4 / 99.2.
+  if (a->D == 64 && static_cast<int64_t>(a->B) * a->H_q * a->q_len * a->N < (int64_t(5) << 20)) return false;
   // One row group per kv head at D = 256 goes to the 32-row decode kernel
   // where that takes the call (4-bit codes, no mask tensor, ...): C3's heads
   // at q_len = 8 over 64K / 128K keys 44.3-44.7 / 72.2-77.0 against
@@ -799,7 +841,8 @@ bool prefill_supports(const qsdpa_decode_args* a) {
   const int kq_bytes = a->D / 4 * a->bits / 8, vp_bytes = a->D / 8 * a->bits / 8;
   if (!aligned_view(a->k_packed, std::min(kq_bytes, 16), 4)) return false;
   if (!aligned_view(a->v_packed, std::min(vp_bytes, 16), 4)) return false;
-  static_assert(128 / PGeo<128>::KPT == 16 && 256 / PGeo<256>::KPT == 16, "K pieces of 16 dims");
+  static_assert(64 / PGeo<64>::KPT == 16 && 128 / PGeo<128>::KPT == 16 && 256 / PGeo<256>::KPT == 16,
+                "K pieces of 16 dims");
   // Row byte offsets up to 4 tiles past the last key stay within 32 bits.
   const int64_t max_sn = std::max({a->k_packed.stride_n * 4, a->v_packed.stride_n * 4, a->k_scales.stride_n * 2,
                                    a->v_scales.stride_n * 2, a->k_biases.stride_n * 2, a->v_biases.stride_n * 2});
@@ -814,14 +857,17 @@ bool prefill_supports(const qsdpa_decode_args* a) {
 // up to the same bounds).  At the C5 chunk (256 row groups) one split; with
 // q_len = 128 (64 groups) 4 splits: 38 against 126 us in one.  (At D = 256,
 // 8 tiles -- the same 256 keys -- made C3's heads at q_len = 16, N = 4096
-// 25.9 instead of 21.3 us.)
+// 25.9 instead of 21.3 us.)  D = 64, whose tiles hold 128 keys: 2 tiles (4
+// tiles, then 1: 32 / 8 heads at q_len = 33 over 4096 keys 20.0, then 16.2,
+// instead of 16.2 us, 300 over 600 keys 15.0 for one split against 19.2 for
+// two and 15.5 for three).
 int prefill_num_splits(const qsdpa_decode_args* a, int cus) {
   const int64_t rows = static_cast<int64_t>(a->H_q / a->H_kv) * a->q_len;
   const int64_t grid = (rows + kPGroupRows - 1) / kPGroupRows * a->H_kv * a->B;
   const int tile = prefill_tile(a->D);
   const int64_t tiles = (static_cast<int64_t>(a->N) + tile - 1) / tile;
   int64_t s = a->num_splits > 0 ? a->num_splits : cus / grid;  // one round of workgroups
-  s = std::min<int64_t>(s, std::max<int64_t>(1, tiles / 4));
+  s = std::min<int64_t>(s, std::max<int64_t>(1, tiles / (a->D == 64 ? 2 : 4)));
   s = std::min<int64_t>(s, kMaxPrefillSplits);
   return static_cast<int>(std::max<int64_t>(s, 1));
 }
@@ -836,6 +882,9 @@ int launch_prefill_mfma(const qsdpa_decode_args* a, int splits, float* part_acc,
     if (a->D == 256) {
       if (a->bits == 4) launch_prefill_gs<Tag, 256, 4>(p, a->group_size, groups, stream, a);
       else launch_prefill_gs<Tag, 256, 8>(p, a->group_size, groups, stream, a);
+    } else if (a->D == 64) {
+      if (a->bits == 4) launch_prefill_gs<Tag, 64, 4>(p, a->group_size, groups, stream, a);
+      else launch_prefill_gs<Tag, 64, 8>(p, a->group_size, groups, stream, a);
     } else {
       if (a->bits == 4) launch_prefill_gs<Tag, 128, 4>(p, a->group_size, groups, stream, a);
       else launch_prefill_gs<Tag, 128, 8>(p, a->group_size, groups, stream, a);

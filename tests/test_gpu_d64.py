@@ -103,6 +103,34 @@ def test_several_positions(device, monkeypatch, dtype, bits, gs):
         _check(q, k, v, bits, gs, mask=keep)
 
 
+@pytest.mark.parametrize("dtype,bits,gs", [(F16, 4, 32), (F16, 8, 64), (BF16, 4, 64), (BF16, 8, 32)])
+def test_prefill(device, dtype, bits, gs):
+    """The prefill kernel (at least 5 * 2^20 query-key pairs): one pass of
+    several rounds, key splits, 128-key tiles cut by the end, a start inside a
+    tile, the causal limit and masks, and a partial row group."""
+    for B, Hq, Hkv, N, L in ((1, 8, 2, 830, 830), (2, 16, 4, 1100, 161), (1, 4, 1, 21000, 66), (1, 24, 8, 767, 300)):
+        assert B * Hq * L * N >= 5 << 20 and Hq // Hkv * L >= 128
+        q, k, v = _inputs(B, Hq, Hkv, N, L, bits, gs, dtype)
+        _check(q, k, v, bits, gs, mask="causal")
+        _check(q, k, v, bits, gs)
+        _check(q, k, v, bits, gs, mask="causal", kv_start=torch.tensor([130, N - L // 2][:B], device=device))
+        if N < 2000:
+            keep = torch.rand(B, Hq if L < 200 else 1, L, N, device=device) < 0.5
+            keep[0, 0, 3] = False
+            _check(q, k, v, bits, gs, mask=keep)
+    q, k, v = _inputs(1, 8, 2, 830, 830, bits, gs, dtype, symmetric=True)
+    _check(q, k, v, bits, gs, mask="causal")
+
+
+@pytest.mark.parametrize("size", [1e-9, 1e-3, 3e6])
+def test_prefill_value_magnitudes(device, size):
+    """bfloat16 V of any magnitude is scaled to the top of float16's range, so
+    small values keep their 8 bits as large ones do."""
+    q, k, v = _inputs(1, 8, 2, 830, 830, 8, 64, BF16)
+    v = (v[0], (v[1].float() * size).to(BF16), (v[2].float() * size).to(BF16))
+    _check(q, k, v, 8, 64, mask="causal")
+
+
 def test_several_positions_on_the_fallback(device, monkeypatch):
     """What the kernel would mask otherwise stays on dequantize + attention."""
     q, k, v = _inputs(2, 4, 2, 300, 3, 4, 32, F16)
@@ -119,13 +147,22 @@ def test_several_positions_on_the_fallback(device, monkeypatch):
 def test_not_a_number_rows(device):
     """A query row of NaN or infinities gives zeros, as the float32 path's
     softmax gives, and leaves the other rows alone."""
-    q, k, v = _inputs(1, 4, 1, 600, 3, 4, 32, F16)
+    _nan_rows(3, 600)
+
+
+def test_not_a_number_rows_prefill(device):
+    _nan_rows(700, 2000)   # one pass
+    _nan_rows(66, 21000)   # key splits
+
+
+def _nan_rows(L, N):
+    q, k, v = _inputs(1, 4, 1, N, L, 4, 32, F16)
     want = mq.fallback_sdpa(q, k, v, bits=4, group_size=32, scale=D ** -0.5)
     q[0, 1, 2, 5] = float("nan")
     q[0, 3, 0, :] = float("inf")
     out = mq.quantized_sdpa(q, k[0], v[0], k[1], v[1], k[2], v[2])
     ref = mq.fallback_sdpa(q, k, v, bits=4, group_size=32, scale=D ** -0.5)
     assert bool((ref[0, 1, 2] == 0).all()) and bool((out[0, 1, 2] == 0).all()) and bool((out[0, 3, 0] == 0).all())
-    rest = torch.ones(4, 3, dtype=torch.bool)
+    rest = torch.ones(4, L, dtype=torch.bool)
     rest[1, 2] = rest[3, 0] = False
     assert float((out[0][rest].float() - want[0][rest].float()).abs().max()) < 2e-3
