@@ -4,7 +4,9 @@ Usage:  python mlx-qsdpa_amd/build_lib.py [--jobs N]
 
 Compiles every csrc/*.hip translation unit for gfx950 and links one shared
 library, mlx_qsdpa_amd/libqsdpa_hip.so, that exports the C ABI declared in
-include/qsdpa.h.  The library depends only on the HIP runtime.
+include/qsdpa.h.  The library depends only on the HIP runtime.  Then the
+torch wrappers' host path (csrc/host.cpp, a CPython extension over the same
+C ABI): mlx_qsdpa_amd/_host.so.
 """
 
 from __future__ import annotations
@@ -69,7 +71,34 @@ def build(jobs: int = 4, verbose: bool = False, extra_flags=(), out: Path | None
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, lib)
+    if out is None:
+        build_host(verbose)
     return lib
+
+
+def build_host(verbose: bool = False) -> Path:
+    """Compile csrc/host.cpp against torch's headers and libqsdpa_hip.so."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    host = PKG / "_host.so"
+    torch_lib = Path(torch.__file__).parent / "lib"
+    rocm = Path(hipcc()).resolve().parents[1]
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-Wno-unused-function",
+           "-D__HIP_PLATFORM_AMD__", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f"-I{sysconfig.get_paths()['include']}", *(f"-isystem{p}" for p in cpp_extension.include_paths()),
+           f"-isystem{rocm / 'include'}", str(CSRC / "host.cpp"), "-o", str(host) + ".tmp",
+           f"-L{torch_lib}", "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", f"-L{PKG}", "-l:libqsdpa_hip.so",
+           f"-L{rocm / 'lib'}", "-lamdhip64", "-Wl,-rpath,$ORIGIN"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed for host.cpp:\n{r.stdout}\n{r.stderr}")
+    os.replace(str(host) + ".tmp", host)
+    return host
 
 
 def main(argv=None) -> int:

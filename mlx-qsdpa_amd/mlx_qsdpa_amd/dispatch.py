@@ -139,18 +139,21 @@ def quantized_sdpa(
         num_splits: optional explicit split count (overrides threshold)
     Returns (B, H_q, qL, D) in q's dtype.
     """
-    # A decode step that repeats an earlier call's geometry relaunches that
-    # call's argument block (the checks below held for it; its shapes and
-    # strides are the block's key).
-    if mask is None and kv_start is None and threshold is None and num_splits is None and q.dim() == 4 \
-            and q.shape[2] == 1 and q.shape[3] in kernels.HEAD_DIMS and bits in (4, 8):
-        both = k_biases is not None and v_biases is not None
-        out = kernels.decode_repeat(q, packed_k, packed_v, k_scales, v_scales, k_biases if both else None,
-                                    v_biases if both else None,
-                                    scale=q.shape[3] ** -0.5 if scale is None else scale, bits=bits,
-                                    group_size=group_size)
-        if out is not None:
-            return out
+    # Calls whose tensors need no conversion go straight to the native host
+    # path, which checks them itself; what it does not take comes back here.
+    if (mask is None or (isinstance(mask, str) and mask == "causal")) \
+            and threshold is None and num_splits is None and q.dim() == 4 and q.shape[3] in kernels.HEAD_DIMS:
+        several = q.shape[2] > 1
+        if not several or q.shape[3] != 64 or (packed_k.dim() == 4 and _d64_in_kernel(
+                mask, kv_start, q.shape[0], q.shape[1], q.shape[2], packed_k.shape[2])):
+            both = k_biases is not None and v_biases is not None
+            out = kernels.decode_repeat(q, packed_k, packed_v, k_scales, v_scales, k_biases if both else None,
+                                        v_biases if both else None,
+                                        scale=q.shape[3] ** -0.5 if scale is None else scale, bits=bits,
+                                        group_size=group_size, kv_start=kv_start,
+                                        causal=several and mask is not None)
+            if out is not None:
+                return out
     B, H_q, qL, D, H_kv, N = _validate(q, packed_k, packed_v, bits, group_size)
     if scale is None:
         scale = D ** -0.5                                          # dispatch.py:86-87

@@ -71,6 +71,20 @@ def to_device(t: torch.Tensor, device) -> torch.Tensor:
     return t.pin_memory().to(device, non_blocking=True)
 
 
+_HOST = None
+
+
+def _host():
+    """The native host path (csrc/host.cpp), loaded on first use.  Its
+    functions return None for what they do not take."""
+    global _HOST
+    if _HOST is None:
+        _lib.load()  # says what to build when it is missing
+        from . import _host as mod
+        _HOST = mod
+    return _HOST
+
+
 _RAW_STREAM = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
@@ -121,6 +135,11 @@ def quantize_into(src: torch.Tensor, dst: tuple, t0: int, bits: int, group_size:
 def quantize_kv_into(keys: torch.Tensor, values: torch.Tensor, kdst: tuple, vdst: tuple, t0: int,
                      bits: int, group_size: int) -> None:
     """quantize_into for the keys and the values of one cache update, in one launch."""
+    if keys.is_cuda:
+        rc = _host().quantize_kv(keys, values, kdst, vdst, t0, bits, group_size, _stream(keys))
+        if rc is not None:
+            _lib.check(rc)
+            return
     if keys.dtype != values.dtype:
         raise ValueError("keys and values must share a dtype")
     keys, ka = _quantize_args(keys, kdst, t0, bits, group_size)
@@ -199,6 +218,25 @@ def requant_window(old: tuple, new: tuple, dst: tuple, n_old: int, keep: int, ro
                                    _view(x), _view(d[0]), _view(d[1]), _view(d[2]))
     _lib.check(_lib.load().qsdpa_requant_window(jobs, 2, _stream(keys)))
     return total
+
+
+def columns(buffers: tuple, n: int) -> tuple:
+    """The first n columns (dim 2) of each of a cache's (B, H, N, W) tensors."""
+    out = _host().columns(buffers, n)
+    return tuple(t[:, :, :n, :] for t in buffers) if out is None else out
+
+
+def grown(keys, values, old, prev, cols, bits, group_size):
+    """Six new cache buffers (packed, scales, biases of the keys and of the
+    values) of `cols` columns in one launch: the first `prev` from `old`,
+    zeros past the new tokens (keys.shape[2] of them, left for the caller to
+    write).  None for tensors it does not take."""
+    if not keys.is_cuda:
+        return None
+    out = _host().grown(keys, values, old, prev, cols, bits, group_size, _stream(keys))
+    if type(out) is int:
+        _lib.check(out)
+    return out
 
 
 class RowMove(NamedTuple):
@@ -433,102 +471,63 @@ class DecodePlan:
         return self.out
 
 
-# Argument blocks of recent decode calls, per thread: a call whose tensors
-# have the geometry of an earlier one -- shapes except the key count, strides,
-# dtypes, pointer alignments, the same scalars and stream -- re-uses that call's validated
-# argument block and workspace, rewriting only the data pointers and the key
-# count (a decode loop over a growing cache hits every step).  The workspace
-# is re-used in the order of the stream it was cached for, so it never races.
+# Split-K workspaces of this thread's decode calls, one per (device, stream):
+# the calls that a thread puts on a stream run in order, so they share one
+# buffer, zero-filled once (the split merge's counters at its start are zero
+# between calls).  At most _WORKSPACES_MAX of them per thread; a dropped one
+# goes back to the allocator, which re-uses it in its stream's order.
 _ARGS = threading.local()
-_ARGS_MAX = 32
+_WORKSPACES_MAX = 32
 
 
-def _cache_key(q, pk, pv, ks, vs, kb, vb, kv_start, scale, bits, group_size, num_splits, causal, stream):
-    """The argument block's key: everything the block encodes except the key
-    count N and the data pointers (but with each pointer's offset from a
-    16-byte boundary), plus the device and stream, or None when
-    the tensors disagree with one another (the full path then raises).  pv
-    must have pk's shape, the scales and biases one shape with pk's (B, H,
-    N)."""
-    sk, ss = pk.shape, ks.shape
-    if pv.shape != sk or vs.shape != ss or ss[:3] != sk[:3] or (kb is not None and kb.shape != ss) \
-            or (vb is not None and vb.shape != ss):
-        return None
-    # The plan (kernel, split count, workspace size) also depends on each
-    # pointer's alignment: a view 2 bytes off its allocation's start can
-    # take another kernel.
-    align = tuple(None if t is None else t.data_ptr() % 16 for t in (q, pk, pv, ks, vs, kb, vb))
-    return (q.shape, q.stride(), q.dtype, sk[0], sk[1], sk[3], pk.dtype, pv.dtype, pk.stride(), pv.stride(), ss[3],
-            ks.dtype, vs.dtype, ks.stride(), vs.stride(), None if kb is None else (kb.dtype, kb.stride()),
-            None if vb is None else (vb.dtype, vb.stride()), None if kv_start is None else kv_start.shape,
-            float(scale), bits, group_size, int(num_splits), bool(causal), q.get_device(), stream, align)
-
-
-def _cached_decode(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start, num_splits,
-                   causal, prof_events):
-    """The decode through a cached argument block; (None, slot) when this
-    geometry has not been seen (the caller then takes the full path and
-    stores its block in `slot`), (None, None) when it cannot be cached."""
-    if not q.is_cuda:
-        return None, None
-    stream = _stream(q)
-    key = _cache_key(q, pk, pv, ks, vs, kb, vb, kv_start, scale, bits, group_size, num_splits, causal, stream)
-    if key is None:
-        return None, None  # inconsistent shapes: the full path raises
-    cache = getattr(_ARGS, "d", None)
-    if cache is None:
-        cache = _ARGS.d = {}
-    hit = cache.get(key)
-    if hit is None:
-        return None, (cache, key)
-    a = hit[0]
-    lib = _lib.load()
-    N = pk.shape[2]
-    a.q.ptr = q.data_ptr()
-    a.k_packed.ptr, a.v_packed.ptr = pk.data_ptr(), pv.data_ptr()
-    a.k_scales.ptr, a.v_scales.ptr = ks.data_ptr(), vs.data_ptr()
-    a.k_biases.ptr = None if kb is None else kb.data_ptr()
-    a.v_biases.ptr = None if vb is None else vb.data_ptr()
-    a.kv_start = None if kv_start is None else kv_start.data_ptr()
-    if N != hit[2]:  # the workspace depends on the geometry and N alone
-        a.N = N
-        ws = _lib.check(lib.qsdpa_decode_workspace_size(ctypes.byref(a), None))
-        if ws > a.workspace_bytes:
-            hit[1] = torch.zeros(ws, dtype=torch.uint8, device=q.device)
-            a.workspace, a.workspace_bytes = hit[1].data_ptr(), ws
-        hit[2] = N
-    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    a.out.ptr = out.data_ptr()
-    a.prof_begin, a.prof_end = prof_events if prof_events is not None else (None, None)
-    _lib.check(lib.qsdpa_decode(ctypes.byref(a), stream))
-    return out, None
-
-
-def decode_repeat(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size):
-    """A decode (no mask, kv_start or explicit split count) that repeats an
-    earlier call's geometry, through its argument block; None when there is
-    no such block or a packed row is not 16-byte aligned (the caller then
-    takes the full path).  Every tensor must be on the GPU (checked)."""
-    if q.is_cuda and pk.is_cuda and pv.is_cuda and ks.is_cuda and vs.is_cuda and (kb is None or kb.is_cuda) \
-            and (vb is None or vb.is_cuda) and q.stride(-1) == 1 and not (pk.data_ptr() | pv.data_ptr()) & 15:
-        out, _ = _cached_decode(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, None, 0, False, None)
-        return out
-    return None
-
-
-# Split-K workspaces of uncached decode calls, one per (device, stream): the
-# calls of a stream run in order, so they can share one buffer, zero-filled
-# once (the split merge's counters at its start are zero between calls).
-_WORKSPACES = {}
-
-
-def _stream_workspace(device, stream, nbytes):
+def _workspace(device, stream, nbytes):
+    """This thread's workspace for `stream` (None if there is none yet and
+    nbytes is 0), grown to nbytes."""
+    held = getattr(_ARGS, "d", None)
+    if held is None:
+        held = _ARGS.d = {}
     key = (device.index, stream)
-    ws = _WORKSPACES.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = torch.zeros(nbytes, dtype=torch.uint8, device=device)
-        _WORKSPACES[key] = ws
+    ws = held.get(key)
+    if nbytes > 0 and (ws is None or ws.numel() < nbytes):
+        if ws is None and len(held) >= _WORKSPACES_MAX:
+            held.pop(next(iter(held)))
+        ws = held[key] = torch.zeros(nbytes, dtype=torch.uint8, device=device)
     return ws
+
+
+def _capture_workspace(device, nbytes):
+    """A workspace for one captured call, from the graph's own memory: the
+    graph replays on it whatever becomes of the shared ones."""
+    ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+    ws[:_TICKET_BYTES].zero_()  # the rest is written before it is read
+    return ws
+
+
+_TICKET_BYTES = 65536
+
+
+def _native_decode(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start, num_splits, causal):
+    """qsdpa_decode through the native host path: the output, its negative
+    code, or None where that does not take the tensors."""
+    stream = _stream(q)
+    ws = _workspace(q.device, stream, 0)
+    fn = _host().decode
+    out = fn(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start, num_splits, causal, ws, stream)
+    if type(out) is int and out > 0:
+        ws = _workspace(q.device, stream, out)
+        out = fn(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start, num_splits, causal, ws, stream)
+    return out
+
+
+def decode_repeat(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size, kv_start=None, causal=False):
+    """A decode without mask or explicit split count whose tensors need no
+    conversion, through the native host path; None for any other call, and
+    for shapes that no kernel takes (the caller then takes the full path,
+    which converts, falls back or raises)."""
+    if not q.is_cuda:
+        return None
+    out = _native_decode(q, pk, pv, ks, vs, kb, vb, float(scale), bits, group_size, kv_start, 0, causal)
+    return out if isinstance(out, torch.Tensor) else None
 
 
 def decode(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size, mask=None, kv_start=None,
@@ -542,8 +541,7 @@ def decode(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size, mask=None, kv_
     ``prof_events``: optional (begin, end) raw hipEvent_t handles recorded
     around the main decode kernel (see qsdpa_decode_args.prof_begin).
 
-    Without a mask, ``out`` or ``workspace``, a call that repeats an earlier
-    call's tensor geometry re-launches that call's argument block.  A
+    Without ``workspace`` the call uses its thread's for the stream.  A
     caller's ``workspace`` (uint8, at least qsdpa_decode_workspace_size
     bytes) must be zero-filled before its first use; the library leaves the
     counters at its start zero after every call, so it can be re-used.
@@ -552,16 +550,15 @@ def decode(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size, mask=None, kv_
     key N - 1 of the caches before the attention (see DecodePlan).
     """
     _require_device(q, pk, pv, ks, vs, kb, vb, mask, kv_start, *(append or ()))
-    slot = None
-    if mask is None and out is None and workspace is None and append is None:
+    if mask is None and out is None and workspace is None and append is None and prof_events is None:
         q = _inner_contig(q)
         if kv_start is not None and (kv_start.dtype != torch.int32 or kv_start.device != q.device
                                      or not kv_start.is_contiguous()):
             kv_start = kv_start.to(device=q.device, dtype=torch.int32).contiguous()
-        res, slot = _cached_decode(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start,
-                                   num_splits, causal, prof_events)
+        res = _native_decode(q, pk, pv, ks, vs, kb, vb, float(scale), bits, group_size, kv_start, int(num_splits),
+                             bool(causal))
         if res is not None:
-            return res
+            return res if isinstance(res, torch.Tensor) else _lib.check(res)
     q = _inner_contig(q)
     if out is None:
         out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
@@ -574,18 +571,14 @@ def decode(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size, mask=None, kv_
     ws = _lib.check(lib.qsdpa_decode_workspace_size(ctypes.byref(a), ctypes.byref(n)))
     if ws > 0:
         if workspace is None or workspace.numel() < ws:
-            workspace = _stream_workspace(q.device, _stream(q), ws)
+            if torch.cuda.is_current_stream_capturing():
+                workspace = _capture_workspace(q.device, ws)
+            else:
+                workspace = _workspace(q.device, _stream(q), ws)
         a.workspace = workspace.data_ptr()
         a.workspace_bytes = ws
     if prof_events is not None:
         a.prof_begin, a.prof_end = prof_events
     _lib.check(lib.qsdpa_decode(ctypes.byref(a), _stream(q)))
     del keep_alive
-    if slot is not None:
-        cache, key = slot
-        if len(cache) >= _ARGS_MAX:
-            cache.pop(next(iter(cache)))
-        if ws <= 0:
-            a.workspace, a.workspace_bytes, workspace = None, 0, None
-        cache[key] = [a, workspace, a.N]
     return out

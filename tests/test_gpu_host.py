@@ -1,0 +1,143 @@
+"""The native host path (csrc/host.cpp) against the wrappers' general path."""
+
+import threading
+
+import pytest
+import torch
+
+import mlx_qsdpa_amd as mq
+from mlx_qsdpa_amd import kernels
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(L=1, B=2, Hq=8, Hkv=2, N=2000, D=128, bits=4, gs=64, dtype=torch.float16, seed=0):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    q = torch.randn(B, Hq, L, D, generator=g, device="cuda").to(dtype)
+    k, v = (kernels.quantize(torch.randn(B, Hkv, N, D, generator=g, device="cuda").to(dtype), gs, bits)
+            for _ in range(2))
+    return dict(q=q, packed_k=k[0], packed_v=v[0], k_scales=k[1], v_scales=v[1], k_biases=k[2], v_biases=v[2],
+                bits=bits, group_size=gs)
+
+
+def _both(monkeypatch, a):
+    """(native path, general path), and whether the native one took the call."""
+    took = []
+    native = kernels._native_decode
+    with monkeypatch.context() as m:
+        m.setattr(kernels, "_native_decode", lambda *x: took.append(native(*x)) or took[-1])
+        got = mq.quantized_sdpa(**a)
+        m.setattr(kernels, "_native_decode", lambda *x: None)
+        want = mq.quantized_sdpa(**a)
+    torch.cuda.synchronize()
+    return got, want, isinstance(took[0], torch.Tensor) if took else False
+
+
+def _off_by_one(t):
+    wide = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+    wide[1:] = t.reshape(-1)
+    return wide[1:].view(t.shape)
+
+
+FORMS = {
+    "plain": ({}, lambda a: a, True),
+    "several": ({"L": 5}, lambda a: dict(a, mask="causal"), True),
+    "symmetric": ({}, lambda a: dict(a, k_biases=None), True),
+    "padded": ({}, lambda a: dict(a, kv_start=torch.tensor([3, 700], dtype=torch.int32, device="cuda")), True),
+    "host_start": ({}, lambda a: dict(a, kv_start=torch.tensor([3, 700])), False),
+    "capacity": ({}, lambda a: {n: x[:, :, :1500] if n[0] in "pkv" else x for n, x in a.items()}, True),
+    "q_strided": ({"L": 3}, lambda a: dict(a, q=a["q"].transpose(1, 2).contiguous().transpose(1, 2)), True),
+    "q_inner": ({}, lambda a: dict(a, q=a["q"].transpose(2, 3).contiguous().transpose(2, 3)), True),
+    "q_2_bytes_off": ({}, lambda a: dict(a, q=_off_by_one(a["q"])), True),
+    "codes_in_odd_rows": ({}, lambda a: dict(a, packed_k=torch.nn.functional.pad(
+        a["packed_k"].view(torch.int32), (1, 0)).view(torch.uint32)[..., 1:]), False),
+    "d256": ({"D": 256, "bits": 8, "dtype": torch.bfloat16}, lambda a: a, True),
+}
+
+
+@pytest.mark.parametrize("form", FORMS)
+def test_native_decode_equals_the_general_path(device, monkeypatch, form):
+    shape, change, native = FORMS[form]
+    print(f"native decode {form}", flush=True)
+    got, want, took = _both(monkeypatch, change(_call(**shape)))
+    assert took == native
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("change,error", [
+    (lambda a: dict(a, v_scales=a["v_scales"][:, :, :-1]), ValueError),
+    (lambda a: dict(a, packed_v=a["packed_v"].view(torch.int32)), ValueError),
+    (lambda a: dict(a, k_scales=a["k_scales"].float()), ValueError),
+    (lambda a: dict(a, kv_start=torch.zeros(3, dtype=torch.int32, device="cuda")), ValueError),
+    (lambda a: dict(a, bits=3), ValueError),
+    (lambda a: dict(a, q=a["q"].cpu()), RuntimeError),
+    (lambda a: dict(a, packed_k=a["packed_k"][:, :, :0], packed_v=a["packed_v"][:, :, :0],
+                    k_scales=a["k_scales"][:, :, :0], v_scales=a["v_scales"][:, :, :0],
+                    k_biases=None, v_biases=None), RuntimeError),
+], ids=["shape", "codes", "scales", "start", "bits", "host", "empty"])
+def test_refusals(device, change, error):
+    with pytest.raises(error):
+        mq.quantized_sdpa(**change(_call()))
+
+
+def test_updates_equal_the_general_path(device, monkeypatch):
+    """Appends and growth: strided new tokens, odd strides of held buffers."""
+    g = torch.Generator(device="cuda").manual_seed(3)
+    steps = [torch.randn(2, 3, n, 64, generator=g, device="cuda").half() for n in (300, 1, 213, 256, 5)]
+
+    def fill():
+        c = mq.BatchQuantizedSDPACache([0, 7], bits=8, group_size=32)
+        for i, x in enumerate(steps):
+            if i == 3:
+                x = x.transpose(2, 3).contiguous().transpose(2, 3)  # strided rows
+            if i == 2:
+                c._keys = tuple(torch.cat([t, t], 1)[:, :3] for t in c._keys)
+            c.update_and_fetch(x, -x)
+        return [t.clone() for t in c._keys + c._values]
+
+    got = fill()
+    monkeypatch.setattr(kernels, "grown", lambda *a: None)
+    real = kernels._host()
+    monkeypatch.setattr(kernels, "_HOST", type("none", (), {"quantize_kv": staticmethod(lambda *a: None),
+                                                           "columns": real.columns}))
+    for a, b in zip(got, fill()):
+        assert a.shape == b.shape and torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
+def test_captured_decode_replays(device):
+    """A captured call keeps a workspace of its own: replays between eager
+    calls that grow and use the shared one give the eager bits."""
+    a, big = _call(N=4000), _call(N=60000, seed=1)
+    want, want_big = mq.quantized_sdpa(**a), mq.quantized_sdpa(**big)
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        mq.quantized_sdpa(**a)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = mq.quantized_sdpa(**a)
+    for _ in range(4):
+        out.zero_()
+        graph.replay()
+        assert torch.equal(mq.quantized_sdpa(**big), want_big)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        kernels._ARGS.d = {}  # the shared workspaces go; the graph's stays
+
+
+def test_threads_on_one_stream(device):
+    """Two threads decoding on the same stream share no workspace."""
+    calls = [_call(N=9000, B=1, seed=s) for s in (5, 6)]
+    want = [mq.quantized_sdpa(**a) for a in calls]
+    torch.cuda.synchronize()
+    bad = []
+
+    def loop(a, w):
+        for _ in range(200):
+            if not torch.equal(mq.quantized_sdpa(**a), w):
+                bad.append(1)
+
+    ts = [threading.Thread(target=loop, args=x) for x in zip(calls, want)]
+    [t.start() for t in ts]
+    [t.join() for t in ts]
+    assert not bad

@@ -397,3 +397,44 @@ def test_plan_capacity_checks():
     # within capacity the plan reaches the device check (these are CPU tensors)
     with pytest.raises(RuntimeError, match="ROCm GPU"):
         kernels.DecodePlan(q, *views[:2], views[2], views[3], views[4], views[5], capacity=cap, **args)
+
+
+# ---- growth ---------------------------------------------------------------
+@pytest.mark.parametrize("held,trim,S,strided", [
+    (300, 0, 213, False),    # trimmed to the held columns: 300 + 256
+    (512, 0, 1, False),      # a multiple of the step: 512 + 256
+    (600, 88, 257, False),   # back to a multiple of the step, in wider buffers: 768 + 512
+    (300, 0, 300, True),     # batch rows that are not the heads' next ones
+], ids=["odd", "full", "stale", "strided"])
+def test_growth_keeps_held_columns_and_zeroes_the_rest(cpu_kernels, rng, held, trim, S, strided):
+    """Buffers after a growing update: the held columns' bits, the new
+    tokens', zeros after them."""
+    B, H, D, step = 2, 3, 64, 256
+    c = pc.BatchQuantizedSDPACache([0] * B, bits=4, group_size=32)
+    c.update_and_fetch(*_kv(rng, B, H, held, D))
+    c.trim(trim)
+    n = held - trim
+    if strided:
+        for name in ("_keys", "_values"):
+            wide = tuple(torch.cat([t, t], dim=1) for t in getattr(c, name))
+            setattr(c, name, tuple(t[:, :H] for t in wide))
+            assert getattr(c, name)[0].stride(0) != H * getattr(c, name)[0].stride(1)
+    before = [t[:, :, :n].clone() for t in c._keys + c._values]
+    cap = c._keys[0].shape[2]
+    cols = (n if n % step else cap) + (S + step - 1) // step * step
+    k, v = _kv(rng, B, H, S, D)
+    c.update_and_fetch(k, v)
+    fresh = pc.BatchQuantizedSDPACache([0] * B, bits=4, group_size=32)
+    want = sum(fresh.update_and_fetch(k, v), ())
+    for t, b, w in zip(c._keys + c._values, before, want):
+        assert t.shape[2] == cols
+        assert torch.equal(t[:, :, :n].contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+        assert torch.equal(t[:, :, n:n + S].contiguous().view(torch.uint8), w.contiguous().view(torch.uint8))
+        assert not t[:, :, n + S:].contiguous().view(torch.uint8).any()
+
+
+def test_growth_rejects_other_shapes(cpu_kernels, rng):
+    c = pc.QuantizedSDPACache(bits=4, group_size=32)
+    c.update_and_fetch(*_kv(rng, 2, 3, 256, 64))
+    with pytest.raises(RuntimeError):
+        c.update_and_fetch(*_kv(rng, 3, 2, 256, 64))
