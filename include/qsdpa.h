@@ -160,7 +160,8 @@ typedef struct {
 } qsdpa_decode_args;
 
 /* Bytes of workspace qsdpa_decode needs for these args (0 for a single
- * pass).  If num_splits_out is not NULL it receives the split count that
+ * pass), and for a prefill under a mask the bytes that let it leave out the
+ * key tiles that the mask rules out (with less it reads every tile).  If num_splits_out is not NULL it receives the split count that
  * qsdpa_decode will use.  Returns a negative QSDPA_ERR_* on bad args.     */
 int64_t qsdpa_decode_workspace_size(const qsdpa_decode_args* args,
                                     int32_t* num_splits_out);

@@ -45,7 +45,8 @@ int launch_decode_mfma(const qsdpa_decode_args* a, int num_splits, float* part_a
 // Defined in prefill_mfma.hip.
 bool prefill_supports(const qsdpa_decode_args* a);
 int prefill_num_splits(const qsdpa_decode_args* a, int cus);
-int launch_prefill_mfma(const qsdpa_decode_args* a, int splits, float* part_acc, float* part_ml,
+int64_t prefill_range_bytes(const qsdpa_decode_args* a);
+int launch_prefill_mfma(const qsdpa_decode_args* a, int splits, float* part_acc, float* part_ml, void* ranges,
                         hipStream_t stream);
 // Defined in decode_rows32.hip (rows32_supports: abi_internal.h).
 int rows32_num_splits(const qsdpa_decode_args* a, int cus);
@@ -228,7 +229,10 @@ bool fused_merge(const qsdpa_decode_args* a, int splits, bool prefill, bool mfma
 
 // Split count: enough workgroups to cover every CU twice, but never fewer
 // than 64 keys per split, and no more than kMaxSplits.
-int decode_plan(const qsdpa_decode_args* a, int* num_splits, int64_t* workspace_bytes) {
+//
+// *workspace_bytes: what the call must have; *ranges_bytes: what it has use
+// for beyond that (a prefill's key ranges under its mask), at the end.
+int decode_plan(const qsdpa_decode_args* a, int* num_splits, int64_t* workspace_bytes, int64_t* ranges_bytes) {
   // Many query positions per kv head: the prefill kernel, with key splits
   // where its row groups alone would leave CUs idle.
   const bool prefill = prefill_supports(a);
@@ -253,12 +257,17 @@ int decode_plan(const qsdpa_decode_args* a, int* num_splits, int64_t* workspace_
   // (U + B, U = splits * B) under the stream-K schedule of a left-padded
   // batch; then that schedule's (first column, count) per sequence.
   *workspace_bytes = splits > 1 ? workspace_layout(a, splits).total : 0;
+  *ranges_bytes = prefill ? prefill_range_bytes(a) : 0;
   return QSDPA_OK;
 }
 
+// Where a call's key ranges lie in its workspace: behind what the call must
+// have, and in a single pass behind the counters, which stay zero.
+int64_t ranges_at(int64_t workspace_bytes) { return std::max(workspace_bytes, kTicketBytes); }
+
 // Launch the decode for validated arguments: the main kernel, then (split-K)
 // the merge, with the partials in `workspace` (decode_plan's layout).
-int run_decode(const qsdpa_decode_args* args, int splits, void* workspace, hipStream_t s) {
+int run_decode(const qsdpa_decode_args* args, int splits, void* workspace, void* ranges, hipStream_t s) {
   // (prof_begin / prof_end ride on the main kernel's own dispatch)
   const bool prefill = prefill_supports(args);
   const bool mfma = mfma_supports(args);
@@ -277,7 +286,7 @@ int run_decode(const qsdpa_decode_args* args, int splits, void* workspace, hipSt
   int rc;
   const bool append_inside = fused_append(args, prefill, mfma);
   if (args->k_new.ptr && !append_inside && (rc = launch_append_quantize(args, s))) return rc;
-  if (prefill) rc = launch_prefill_mfma(args, splits, part_acc, part_ml, s);
+  if (prefill) rc = launch_prefill_mfma(args, splits, part_acc, part_ml, ranges, s);
   else if (mfma && rows32_supports(args)) rc = launch_decode_rows32(args, splits, part_acc, part_ml, units, sched, s);
   else if (mfma)
     rc = launch_decode_mfma(args, splits, part_acc, part_ml, units, sched,
@@ -340,11 +349,11 @@ int64_t qsdpa_decode_workspace_size(const qsdpa_decode_args* args, int32_t* num_
   int rc = validate_decode(args);
   if (rc) return rc;
   int splits = 1;
-  int64_t ws = 0;
-  rc = decode_plan(args, &splits, &ws);
+  int64_t ws = 0, extra = 0;
+  rc = decode_plan(args, &splits, &ws, &extra);
   if (rc) return rc;
   if (num_splits_out) *num_splits_out = splits;
-  return ws;
+  return extra > 0 ? ranges_at(ws) + extra : ws;
 }
 
 int qsdpa_decode(const qsdpa_decode_args* args, void* stream) {
@@ -352,8 +361,8 @@ int qsdpa_decode(const qsdpa_decode_args* args, void* stream) {
   int rc = validate_decode(args);
   if (rc) return rc;
   int splits = 1;
-  int64_t ws = 0;
-  rc = decode_plan(args, &splits, &ws);
+  int64_t ws = 0, extra = 0;
+  rc = decode_plan(args, &splits, &ws, &extra);
   if (rc) return rc;
   if (splits > 1) {
     if (!args->workspace || static_cast<int64_t>(args->workspace_bytes) < ws)
@@ -361,7 +370,12 @@ int qsdpa_decode(const qsdpa_decode_args* args, void* stream) {
                   static_cast<long long>(ws), static_cast<long long>(args->workspace_bytes));
     if (!aligned(args->workspace, 16)) return fail(QSDPA_ERR_INVALID, "workspace not 16-byte aligned");
   }
-  return run_decode(args, splits, args->workspace, static_cast<hipStream_t>(stream));
+  // A prefill whose workspace ends before the key ranges takes its mask as it is.
+  void* ranges = nullptr;
+  if (extra > 0 && args->workspace && static_cast<int64_t>(args->workspace_bytes) >= ranges_at(ws) + extra &&
+      aligned(args->workspace, 16))
+    ranges = static_cast<uint8_t*>(args->workspace) + ranges_at(ws);
+  return run_decode(args, splits, args->workspace, ranges, static_cast<hipStream_t>(stream));
 }
 
 int qsdpa_decode_noalloc(const qsdpa_decode_args* args, void* stream) {
@@ -369,10 +383,14 @@ int qsdpa_decode_noalloc(const qsdpa_decode_args* args, void* stream) {
   int rc = validate_decode(args);
   if (rc) return rc;
   int splits = 1;
-  int64_t ws = 0;
-  rc = decode_plan(args, &splits, &ws);
+  int64_t ws = 0, extra = 0;
+  rc = decode_plan(args, &splits, &ws, &extra);
   if (rc) return rc;
-  void* scratch_ptr = nullptr;
+  void *scratch_ptr = nullptr, *ranges = nullptr;
+  if (extra > 0 && ranges_at(ws) + extra <= static_cast<int64_t>(kScratchBytes)) {
+    if ((rc = scratch_address(&scratch_ptr))) return rc;
+    ranges = static_cast<uint8_t*>(scratch_ptr) + ranges_at(ws);
+  }
   if (splits > 1) {
     if (ws > static_cast<int64_t>(kScratchBytes))
       return fail(QSDPA_ERR_WORKSPACE,
@@ -381,7 +399,7 @@ int qsdpa_decode_noalloc(const qsdpa_decode_args* args, void* stream) {
                   static_cast<long long>(ws), static_cast<long long>(kScratchBytes));
     if ((rc = scratch_address(&scratch_ptr))) return rc;
   }
-  return run_decode(args, splits, scratch_ptr, static_cast<hipStream_t>(stream));
+  return run_decode(args, splits, scratch_ptr, ranges, static_cast<hipStream_t>(stream));
 }
 
 int qsdpa_quantize(const qsdpa_quantize_args* a, void* stream) {

@@ -66,6 +66,10 @@ struct MfmaParams {
   // v % G); a block takes 16 consecutive rows.
   int qL, causal;
   int64_t q_sq, o_sq, m_sq;  // position strides of q, out and the mask
+  // Prefill with a mask tensor (null = every key): the keys that it leaves
+  // each row group, per key chunk (mask_range_kernel).
+  int2* ranges;
+  int range_chunks;
   // Folded append (null = none): the new K / V rows [B, H_kv, 1, D], which
   // the workgroup that reads key N - 1 quantizes into that key first.
   const uint16_t* knew;
@@ -324,6 +328,8 @@ inline MfmaParams mfma_params(const qsdpa_decode_args* a, int num_splits, float*
   p.units = 0;
   p.sched = nullptr;
   p.tickets = nullptr;
+  p.ranges = nullptr;
+  p.range_chunks = 0;
   p.knew = p.vnew = nullptr;
   p.knew_sb = p.knew_sh = p.vnew_sb = p.vnew_sh = 0;
   return p;

@@ -345,6 +345,102 @@ struct Prefill {
   }
 };
 
+// ---- The range of keys that a mask tensor leaves (MASK) ----
+// A causal, windowed or left-padded mask leaves many tiles without a key for
+// any row of a group (half of a prompt's), which the kernel would
+// dequantize, multiply and mask like the others.  mask_range_kernel reads the
+// mask once, and a row group then runs from the tile of its first attended
+// key to that of its last.  Only masks whose keys are adjacent and whose rows
+// are shared by the heads: one pass over one head's mask then serves all of
+// them.  Memory-latency bound; 2.5 us for 8 masks of 500 x 1500 bools.
+//
+// At that chunk (8 sequences of 32 / 8 heads, 8-bit bf16; attention alone)
+// 137.5 us under the batch cache's mask against 200 over every tile, 193 under
+// one causal mask for all.  The same look inside the prefill kernel, by each
+// workgroup for itself, took 176, a list there of the tiles with an attended
+// key 164 (and 249 instead of 200 for a mask with holes everywhere: an index
+// from the LDS per tile).
+__host__ __device__ constexpr int mask_bytes(int kind) {
+  return kind == QSDPA_BOOL ? 1 : kind == QSDPA_F32 ? 4 : 2;
+}
+
+// Whether a word of mask values attends any key (mask_values' -infinity).
+template <int KIND>
+__device__ __forceinline__ bool mask_word(uint32_t w) {
+  if constexpr (KIND == QSDPA_BOOL) {
+    return w != 0u;
+  } else if constexpr (KIND == QSDPA_F32) {
+    return !(__builtin_bit_cast(float, w) * kLog2e == -__builtin_huge_valf());
+  } else {
+    bool any = false;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint16_t x = static_cast<uint16_t>(w >> (16 * h));
+      any |= !((KIND == QSDPA_F16 ? f16_bits_to_f32(x) : bf16_bits_to_f32(x)) * kLog2e == -__builtin_huge_valf());
+    }
+    return any;
+  }
+}
+
+// Grid (key chunks, row groups, B): the first attended key of the group's
+// positions in the chunk and one past the last, in columns of 16 bytes of
+// mask, to ranges[(b * groups + group) * chunks + chunk] (0, 0: none).  A
+// thread takes a column down its share of the rows, eight loads in flight.
+// (Rows start at any byte: the loads are unaligned ones.)
+template <int KIND>
+__global__ __launch_bounds__(512) void mask_range_kernel(MfmaParams p, int chunk) {
+  constexpr int ES = mask_bytes(KIND), E = 16 / ES;  // keys per column
+  constexpr int U = 8;
+  __shared__ int s_lo, s_hi;
+  const int tid = threadIdx.x;
+  if (tid == 0) {
+    s_lo = 0x7FFFFFFF;
+    s_hi = 0;
+  }
+  __syncthreads();
+  const int rows = p.G * p.qL, v_first = blockIdx.y * kPGroupRows;
+  const int v_last = min(v_first + kPGroupRows, rows) - 1;
+  const int iq0 = v_first / p.G;
+  const int R = p.m_sq != 0 ? v_last / p.G - iq0 + 1 : 1;
+  const int k0 = blockIdx.x * chunk, k1 = min(k0 + chunk, p.N);
+  const uint8_t* base = static_cast<const uint8_t*>(p.mask) +
+                        (static_cast<int64_t>(blockIdx.z) * p.m_sb + static_cast<int64_t>(iq0) * p.m_sq) * ES;
+  const int cols = (k1 - k0 + E - 1) / E;
+  int side = 64;  // threads side by side over the columns, the others share the rows
+  while (side < cols && side < 512) side *= 2;
+  const int shares = 512 / side, share = tid / side;
+  int lo = 0x7FFFFFFF, hi = 0;
+  for (int c = tid % side; c < cols; c += side) {
+    const int k = min(k0 + c * E, p.N - E);  // the last column ends with the row
+    bool any = k < 0;                        // fewer keys than a column: not looked at
+    if (k >= 0) {
+      for (int r0 = share; r0 < R && !any; r0 += U * shares) {
+        u4 w[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)  // (rows past the last repeat it)
+          __builtin_memcpy(&w[u], base + (static_cast<int64_t>(min(r0 + u * shares, R - 1)) * p.m_sq + k) * ES, 16);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) any |= mask_word<KIND>(w[u][i]);
+      }
+    }
+    if (any) {
+      lo = min(lo, max(k, 0));
+      hi = max(hi, max(k, 0) + E);
+    }
+  }
+  if (hi > 0) {
+    atomicMin(&s_lo, lo);
+    atomicMax(&s_hi, hi);
+  }
+  __syncthreads();
+  if (tid == 0) {
+    const int64_t at = (static_cast<int64_t>(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    p.ranges[at] = s_hi > 0 ? int2{s_lo, min(s_hi, p.N)} : int2{0, 0};
+  }
+}
+
 // Parameters beyond the decode's: none; the same MfmaParams (q_len > 1).
 // MASK: calls with a mask tensor (an instantiation of their own, so that the
 // unmasked kernel carries none of the mask code).
@@ -367,20 +463,30 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
   // robin, so the work of workgroup id w goes to XCD w % 8 in consecutive
   // runs: the row groups of one (batch, kv head) share one XCD's L2.
   //
-  // Causal calls of several rounds of workgroups: a row group's work grows
-  // with its position, so each head's groups run from the longest down (the
-  // last workgroups to start are then the shortest), and where the heads do
-  // not divide evenly over the XCDs the heads alternate instead, so that no
-  // XCD holds only long groups.  A prompt of 3000 tokens (32 / 8 heads,
-  // 4-bit; 752 workgroups), with its cache update: 142.6 us against 156.5
-  // with the shortest groups first.
+  // Causal calls (and those with a mask tensor, which mostly is causal too) of
+  // several rounds of workgroups: a row group's work grows with its position,
+  // so each head's groups run from the longest down (the last workgroups to
+  // start are then the shortest), and where the heads do not divide evenly
+  // over the XCDs the heads alternate instead, so that no XCD holds only long
+  // groups.  A prompt of 3000 tokens (32 / 8 heads, 4-bit; 752 workgroups),
+  // with its cache update: 142.6 us against 156.5 with the shortest groups
+  // first.  Where the sequences' key ranges may differ (a start each, or a
+  // mask), an XCD takes every eighth head, so that it does not hold one
+  // sequence alone: 8 sequences of 500 x 1500 (32 / 8 heads, 8-bit bf16) under
+  // the batch cache's mask 137.5 us against 195 in runs, with a start each and
+  // the causal limit 134 against 154; a mask with random holes everywhere,
+  // whose rows then pass through every XCD's L2, takes 218 against 207.
   const int total = gridDim.x;
   const int heads = p.Hkv * p.B;
   const int S = p.num_splits;
+  const bool uneven = p.B > 1 && (MASK || p.kv_start);
   int w = blockIdx.x, split = 0, grp, head;
-  if (p.causal && S == 1 && heads % 8 != 0) {
+  if ((p.causal || MASK || uneven) && S == 1 && heads % 8 != 0) {
     head = w % heads;
     grp = w / heads;
+  } else if (uneven && S == 1) {
+    head = w % 8 + 8 * (w / 8 / groups_per_head);
+    grp = w / 8 % groups_per_head;
   } else {
     if (total % 8 == 0) w = (w % 8) * (total / 8) + w / 8;
     split = w % S;
@@ -388,7 +494,7 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
     grp = w % groups_per_head;
     head = w / groups_per_head;
   }
-  if (p.causal) grp = groups_per_head - 1 - grp;
+  if (p.causal || MASK) grp = groups_per_head - 1 - grp;
   const int kvh = head % p.Hkv;
   const int b = head / p.Hkv;
 
@@ -400,10 +506,24 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
   const int n_end = p.causal ? min(p.N, max(0, p.N - p.qL + (v_first + nrows - 1) / p.G + 1)) : p.N;
   const int len = max(n_end - s0, 0);
   constexpr int kTile = PG::Tile, NT = PG::NT, NU = PG::NU, KS = PG::KS;
-  const int T_all = (len + kTile - 1) / kTile;
-  // This split's tiles: [j_base, j_base + T) of the group's T_all.
-  const int j_base = static_cast<int>(static_cast<int64_t>(split) * T_all / S);
-  const int T = static_cast<int>(static_cast<int64_t>(split + 1) * T_all / S) - j_base;
+  int T_all = (len + kTile - 1) / kTile, j_first = 0;
+  if constexpr (MASK) {
+    if (p.ranges) {  // [j_first, j_first + T_all): the tiles that the mask leaves
+      const int2* rg = p.ranges + (static_cast<int64_t>(b) * groups_per_head + grp) * p.range_chunks;
+      const int2 x = lane < p.range_chunks ? rg[lane] : int2{0, 0};
+      const uint64_t m = __builtin_amdgcn_ballot_w64(x.y > 0);
+      int lo = 0, hi = 0;
+      if (m) {
+        lo = __builtin_amdgcn_readlane(x.x, static_cast<int>(__builtin_ctzll(m)));
+        hi = __builtin_amdgcn_readlane(x.y, 63 - static_cast<int>(__builtin_clzll(m)));
+      }
+      j_first = max(lo - s0, 0) / kTile;
+      T_all = max(min(T_all, (max(hi - s0, 0) + kTile - 1) / kTile) - j_first, 0);
+    }
+  }
+  // This split's tiles: [j_base, j_base + T) of the group's.
+  const int j_base = j_first + static_cast<int>(static_cast<int64_t>(split) * T_all / S);
+  const int T = j_first + static_cast<int>(static_cast<int64_t>(split + 1) * T_all / S) - j_base;
 
   // The lane's row: v = v_first + 16 wave + r (clamped to the last real row).
   int n_lane, n_wave;  // the lane's key limit; the wave's smallest
@@ -767,6 +887,19 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
   }
 }
 
+// Key chunks of mask_range_kernel: at most 64 (a wave's lanes read them), of
+// at least 1024 keys, in whole columns of 16.
+int range_chunk(int N) { return std::max(1024, ((N + 63) / 64 + 15) / 16 * 16); }
+
+void launch_mask_range(const MfmaParams& p, int groups, hipStream_t stream) {
+  const int chunk = range_chunk(p.N);
+  void (*k)(MfmaParams, int) = p.mask_kind == QSDPA_BOOL ? mask_range_kernel<QSDPA_BOOL>
+                               : p.mask_kind == QSDPA_F16 ? mask_range_kernel<QSDPA_F16>
+                               : p.mask_kind == QSDPA_BF16 ? mask_range_kernel<QSDPA_BF16>
+                                                           : mask_range_kernel<QSDPA_F32>;
+  hipLaunchKernelGGL(k, dim3(p.range_chunks, groups, p.B), dim3(512), 0, stream, p, chunk);
+}
+
 template <typename Tag, int D, int BITS, bool MASK>
 void launch_prefill_mask(const MfmaParams& p, int gs, int groups, hipStream_t stream, const qsdpa_decode_args* a) {
   const dim3 grid(groups * p.Hkv * p.B * p.num_splits);
@@ -872,10 +1005,26 @@ int prefill_num_splits(const qsdpa_decode_args* a, int cus) {
   return static_cast<int>(std::max<int64_t>(s, 1));
 }
 
-int launch_prefill_mfma(const qsdpa_decode_args* a, int splits, float* part_acc, float* part_ml,
+// Workspace bytes of the row groups' key ranges under the call's mask; 0
+// where the kernel takes the mask as it is (heads with masks of their own,
+// keys that are not adjacent, more groups than a grid dimension holds).
+int64_t prefill_range_bytes(const qsdpa_decode_args* a) {
+  if (!a->mask.ptr || a->mask.stride_n != 1 || a->mask.stride_h != 0) return 0;
+  const int64_t groups = (static_cast<int64_t>(a->H_q / a->H_kv) * a->q_len + kPGroupRows - 1) / kPGroupRows;
+  if (groups > 65535 || a->B > 65535) return 0;
+  const int64_t chunks = (a->N + range_chunk(a->N) - 1) / range_chunk(a->N);
+  return (groups * a->B * chunks * 8 + 255) / 256 * 256;
+}
+
+int launch_prefill_mfma(const qsdpa_decode_args* a, int splits, float* part_acc, float* part_ml, void* ranges,
                         hipStream_t stream) {
   MfmaParams p = mfma_params(a, splits, part_acc, part_ml);
   const int groups = (p.G * p.qL + kPGroupRows - 1) / kPGroupRows;
+  if (ranges) {
+    p.ranges = static_cast<int2*>(ranges);
+    p.range_chunks = (p.N + range_chunk(p.N) - 1) / range_chunk(p.N);
+    launch_mask_range(p, groups, stream);
+  }
   const bool f16 = a->dtype == QSDPA_F16;
   auto bits = [&](auto tag) {
     using Tag = decltype(tag);

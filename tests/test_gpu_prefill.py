@@ -387,3 +387,45 @@ def test_prefill_split_merge_unaligned_out(device, dtype):
     torch.cuda.synchronize()
     assert torch.equal(out, ref)
     assert bool((wide[..., 0] == 0).all()) and bool((wide[..., 129] == 0).all())
+
+
+def _block_mask(B, L, N, seed):
+    """A bool mask whose rows see a band of keys, with random holes in some
+    blocks and others whole or empty; one sequence is left-padded, the first
+    rows of another see nothing."""
+    g = torch.Generator().manual_seed(seed)
+    rows, cols = torch.arange(L)[:, None] + (N - L), torch.arange(N)[None, :]
+    keep = ((cols <= rows) & (cols > rows - N // 2)).repeat(B, 1, 1, 1)
+    holes = torch.rand(B, 1, L, N, generator=g) < 0.6
+    keep = torch.where((cols // 100) % 3 == 0, keep & holes, keep)
+    keep[-1, :, :, : N // 3] = False
+    keep[0, :, : L // 2] = False
+    return keep
+
+
+@pytest.mark.parametrize("D,bits,gs,dtype", [(128, 4, 64, torch.float16), (128, 8, 128, torch.bfloat16),
+                                             (256, 4, 32, torch.float16), (256, 8, 64, torch.bfloat16),
+                                             (64, 4, 32, torch.float16), (64, 8, 64, torch.bfloat16)])
+@pytest.mark.parametrize("B,Hq,Hkv,N,L", [(2, 32, 8, 1001, 333), (1, 16, 2, 4099, 130)], ids=["rounds", "splits"])
+def test_prefill_skips_masked_tiles(device, D, bits, gs, dtype, B, Hq, Hkv, N, L):
+    """Masks that rule out whole tiles at either end of a row group's keys:
+    bool and additive, odd row lengths, one mask row for all positions,
+    per-head masks (taken as they are), with a start and the causal limit; an
+    all-masked row group gives zeros."""
+    if D == 64:
+        Hq = Hkv * 16  # enough pairs for the prefill kernel
+    q, kq, vq = _inputs(B, Hq, Hkv, N, L, bits, gs, dtype, seed=N, D=D)
+    keep = _block_mask(B, L, N, seed=L).to(device)
+    print(f"prefill block mask D={D} {dtype} N={N} L={L}", flush=True)
+    _check(q, kq, vq, bits, gs, "bool", mask=keep)
+    ks = torch.tensor([77, 400][:B], dtype=torch.int32, device=device)
+    _check(q, kq, vq, bits, gs, "bool, start, causal", mask=keep, kv_start=ks, causal=True)
+    for t in (dtype, torch.float32):
+        add = torch.where(keep, 0.0, float("-inf")).to(t)
+        add[..., 100:140] += 2.0
+        _check(q, kq, vq, bits, gs, f"additive {t}", mask=add)
+    _check(q, kq, vq, bits, gs, "one row", mask=keep[:, :, -1:])
+    heads = keep & (torch.rand(1, Hq, 1, N, generator=torch.Generator().manual_seed(4)) < 0.9).to(device)
+    _check(q, kq, vq, bits, gs, "per head", mask=heads)
+    _check(q, kq, vq, bits, gs, "nothing", mask=torch.zeros_like(keep))
+    _check(q, kq, vq, bits, gs, "everything", mask=torch.ones_like(keep), causal=True)
