@@ -34,6 +34,8 @@
  *                       + trim + quantize (cache.py:593-634, 813-857).
  *   qsdpa_move_rows  <- the batch caches' slicing / padding / concatenation
  *                       (cache.py:46-51, 337-348, 378-492, 868-1010).
+ *   qsdpa_rotate     <- (no counterpart) the rotary positions of the layer
+ *                       that calls the caches.
  */
 #ifndef QSDPA_H_
 #define QSDPA_H_
@@ -296,6 +298,23 @@ typedef struct {
 } qsdpa_row_move;
 
 int qsdpa_move_rows(const qsdpa_row_move* moves, int32_t count, void* stream);
+
+/*
+ * Rotary positions of a layer's queries [B, H_q, L, D] and keys [B, H_kv, L,
+ * D] in one launch (per 64 sequences): elements i and i + D / 2 of a head turn
+ * by (start[b] + l) * theta^(-2 i / D), computed in float32 and rounded to
+ * dtype (QSDPA_F16 / QSDPA_BF16).  start is HOST memory (B values), read
+ * before the call returns.  D even, at most 1024; the outputs overlap nothing.
+ */
+typedef struct {
+  int32_t B, H_q, H_kv, L, D;
+  int32_t dtype;
+  float theta;
+  const int64_t* start;
+  qsdpa_view q, k, q_out, k_out;
+} qsdpa_rotate_args;
+
+int qsdpa_rotate(const qsdpa_rotate_args* args, void* stream);
 
 /* Thread-local message describing the last error ("" if none). */
 const char* qsdpa_last_error(void);

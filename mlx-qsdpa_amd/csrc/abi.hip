@@ -490,6 +490,22 @@ int qsdpa_move_rows(const qsdpa_row_move* moves, int32_t count, void* stream) {
   return launch_move_rows(moves, count, static_cast<hipStream_t>(stream));
 }
 
+int qsdpa_rotate(const qsdpa_rotate_args* a, void* stream) {
+  clear_error();
+  if (!a) return fail(QSDPA_ERR_INVALID, "null args");
+  if (a->B < 0 || a->H_q < 0 || a->H_kv < 0 || a->L < 0 || a->D < 2 || a->D % 2 != 0)
+    return fail(QSDPA_ERR_INVALID, "bad shape B=%d H_q=%d H_kv=%d L=%d D=%d", a->B, a->H_q, a->H_kv, a->L, a->D);
+  // Heads times pieces of a token, one element each at least, in an int.
+  if (a->D > 1024 || static_cast<int64_t>(std::max(a->H_q, a->H_kv)) * a->D > INT32_MAX)
+    return fail(QSDPA_ERR_UNSUPPORTED, "D=%d with %d / %d heads is too large", a->D, a->H_q, a->H_kv);
+  if (a->dtype != QSDPA_F16 && a->dtype != QSDPA_BF16)
+    return fail(QSDPA_ERR_INVALID, "dtype must be QSDPA_F16 or QSDPA_BF16, got %d", a->dtype);
+  if (a->B == 0 || a->L == 0) return QSDPA_OK;
+  if (!a->start || (a->H_q > 0 && (!a->q.ptr || !a->q_out.ptr)) || (a->H_kv > 0 && (!a->k.ptr || !a->k_out.ptr)))
+    return fail(QSDPA_ERR_INVALID, "null pointer");
+  return launch_rotate(a, static_cast<hipStream_t>(stream));
+}
+
 int qsdpa_dequantize(const qsdpa_dequantize_args* a, void* stream) {
   clear_error();
   if (!a) return fail(QSDPA_ERR_INVALID, "null args");

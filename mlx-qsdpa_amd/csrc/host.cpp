@@ -20,7 +20,11 @@
 
 #include <ATen/ATen.h>
 #include <ATen/TensorSubclassLikeUtils.h>
+#include <c10/core/GradMode.h>
 #include <hip/hip_runtime_api.h>
+
+#include <algorithm>
+#include <vector>
 
 #include "../../include/qsdpa.h"
 
@@ -276,6 +280,63 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// A tensor that no gradient, of either mode, is taken through.
+bool constant(const at::Tensor& t) {
+  return !(c10::GradMode::is_enabled() && t.requires_grad()) && !t._fw_grad(0).defined();
+}
+
+// rotate(q, k, start, theta, stream): q and k [B, H, L, D] with the rotary
+// positions start (an int, or a CPU tensor of 1 or B of them) + l, as a tuple
+// of contiguous tensors; the negative code of qsdpa_rotate; or None.
+PyObject* rotate(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  int64_t stream, first = 0;
+  if (n != 5 || !PyFloat_Check(a[3]) || !as_int(a[4], stream)) Py_RETURN_NONE;
+  const at::Tensor *q = plain4(a[0]), *k = plain4(a[1]);
+  if (!q || !k || !constant(*q) || !constant(*k) || q->device() != k->device() || dtype_of(*q) < 0 ||
+      k->scalar_type() != q->scalar_type())
+    Py_RETURN_NONE;
+  int device = -1;
+  if (hipGetDevice(&device) != hipSuccess || device != q->device().index()) Py_RETURN_NONE;
+  const int64_t B = q->size(0), Hq = q->size(1), L = q->size(2), D = q->size(3), Hkv = k->size(1);
+  if (B < 1 || L < 1 || D < 2 || D % 2 || D > 1024 || !shaped(*k, B, Hkv, L, D) || !fits32({B, Hq * D, Hkv * D, L}))
+    Py_RETURN_NONE;
+  std::vector<int64_t> start(B);
+  if (THPVariable_CheckExact(a[2])) {
+    const at::Tensor& t = THPVariable_Unpack(a[2]);
+    if (!t.device().is_cpu() || t.layout() != at::kStrided || at::isTensorSubclassLike(t) || t.dim() > 1 ||
+        t.scalar_type() != at::kLong || (t.numel() != 1 && t.numel() != B))
+      Py_RETURN_NONE;
+    const int64_t* x = t.data_ptr<int64_t>();
+    const int64_t step = t.dim() == 1 && t.numel() == B ? t.stride(0) : 0;
+    for (int64_t b = 0; b < B; ++b) start[b] = x[b * step];
+  } else if (as_int(a[2], first)) {
+    std::fill(start.begin(), start.end(), first);
+  } else {
+    Py_RETURN_NONE;
+  }
+  at::Tensor out[2] = {at::empty({B, Hq, L, D}, q->options().requires_grad(false)),
+                       at::empty({B, Hkv, L, D}, q->options().requires_grad(false))};
+  qsdpa_rotate_args x = {};
+  x.B = B; x.H_q = Hq; x.H_kv = Hkv; x.L = L; x.D = D;
+  x.dtype = dtype_of(*q);
+  x.theta = static_cast<float>(PyFloat_AS_DOUBLE(a[3]));
+  x.start = start.data();
+  x.q = view(*q); x.k = view(*k);
+  x.q_out = view(out[0]); x.k_out = view(out[1]);
+  const int rc = qsdpa_rotate(&x, stream_of(stream));
+  if (rc) return PyLong_FromLong(rc);
+  THPObjectPtr pair(PyTuple_New(2));
+  if (!pair) return nullptr;
+  for (int i = 0; i < 2; ++i) {
+    PyObject* o = THPVariable_Wrap(std::move(out[i]));
+    if (!o) return nullptr;
+    PyTuple_SET_ITEM(pair.get(), i, o);
+  }
+  return pair.release();
+  END_HANDLE_TH_ERRORS
+}
+
 template <PyObject* (*F)(PyObject*, PyObject* const*, Py_ssize_t)>
 PyCFunction fast() {
   return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(F));
@@ -286,6 +347,7 @@ PyMethodDef methods[] = {
     {"columns", fast<columns>(), METH_FASTCALL, nullptr},
     {"grown", fast<grown>(), METH_FASTCALL, nullptr},
     {"decode", fast<decode>(), METH_FASTCALL, nullptr},
+    {"rotate", fast<rotate>(), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 

@@ -239,6 +239,19 @@ def grown(keys, values, old, prev, cols, bits, group_size):
     return out
 
 
+def rotate(q, k, start, theta):
+    """q and k [B, H, L, D] turned to the rotary positions start + l in one
+    launch (csrc/rotate.hip), contiguous; `start` an int or a CPU tensor of
+    one per sequence.  None for what the kernel does not take, and where a
+    gradient or a trace goes through q or k."""
+    if not q.is_cuda or torch.jit.is_tracing() or torch.compiler.is_compiling():
+        return None
+    out = _host().rotate(q, k, start, theta, _stream(q))
+    if type(out) is int:
+        _lib.check(out)
+    return out
+
+
 class RowMove(NamedTuple):
     """Fill token columns [dst_col, dst_col + tokens) of batch row `dst_row` of
     a (B, H, N, W) buffer, every head: the columns dst_col + [copy_begin,
