@@ -34,6 +34,8 @@
  *                       + trim + quantize (cache.py:593-634, 813-857).
  *   qsdpa_move_rows  <- the batch caches' slicing / padding / concatenation
  *                       (cache.py:46-51, 337-348, 378-492, 868-1010).
+ *   qsdpa_causal_mask <- the comparisons of _create_causal_mask
+ *                       (cache.py:15-43).
  *   qsdpa_rotate     <- (no counterpart) the rotary positions of the layer
  *                       that calls the caches.
  */
@@ -298,6 +300,22 @@ typedef struct {
 } qsdpa_row_move;
 
 int qsdpa_move_rows(const qsdpa_row_move* moves, int32_t count, void* stream);
+
+/*
+ * The mask of a causal pass, out[b, i, k] = start[b] + i - window < k <=
+ * start[b] + i and k >= pad[b], as contiguous [B, N, total] bytes of 0 or 1,
+ * in one launch (per 64 sequences).  start and pad (NULL: no padding) are HOST memory of B values,
+ * read before the call returns; they and the window within +-2^34.
+ */
+typedef struct {
+  int32_t B, N, total;
+  int64_t window;
+  const int64_t* start;
+  const int64_t* pad;
+  uint8_t* out;
+} qsdpa_causal_mask_args;
+
+int qsdpa_causal_mask(const qsdpa_causal_mask_args* args, void* stream);
 
 /*
  * Rotary positions of a layer's queries [B, H_q, L, D] and keys [B, H_kv, L,

@@ -490,6 +490,21 @@ int qsdpa_move_rows(const qsdpa_row_move* moves, int32_t count, void* stream) {
   return launch_move_rows(moves, count, static_cast<hipStream_t>(stream));
 }
 
+int qsdpa_causal_mask(const qsdpa_causal_mask_args* a, void* stream) {
+  clear_error();
+  if (!a) return fail(QSDPA_ERR_INVALID, "null args");
+  if (a->B < 0 || a->N < 0 || a->total < 0)
+    return fail(QSDPA_ERR_INVALID, "bad shape B=%d N=%d total=%d", a->B, a->N, a->total);
+  if (a->B == 0 || a->N == 0 || a->total == 0) return QSDPA_OK;
+  if (!a->start || !a->out) return fail(QSDPA_ERR_INVALID, "null pointer");
+  constexpr int64_t kLimit = int64_t(1) << 34;
+  auto outside = [](int64_t x) { return x < -kLimit || x > kLimit; };
+  bool bad = outside(a->window);
+  for (int b = 0; b < a->B; ++b) bad = bad || outside(a->start[b]) || (a->pad && outside(a->pad[b]));
+  if (bad) return fail(QSDPA_ERR_INVALID, "positions, padding and window must lie within +-2^34");
+  return launch_causal_mask(a, static_cast<hipStream_t>(stream));
+}
+
 int qsdpa_rotate(const qsdpa_rotate_args* a, void* stream) {
   clear_error();
   if (!a) return fail(QSDPA_ERR_INVALID, "null args");

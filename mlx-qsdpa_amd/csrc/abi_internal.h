@@ -50,6 +50,7 @@ int launch_quantize(const qsdpa_quantize_args* const* jobs, int count, hipStream
 int launch_dequantize(const qsdpa_dequantize_args* a, hipStream_t stream);
 int launch_requant(const qsdpa_requant_args* const* jobs, int count, hipStream_t stream);
 int launch_move_rows(const qsdpa_row_move* moves, int count, hipStream_t stream);
+int launch_causal_mask(const qsdpa_causal_mask_args* a, hipStream_t stream);
 int launch_rotate(const qsdpa_rotate_args* a, hipStream_t stream);
 int launch_decode(const qsdpa_decode_args* a, int num_splits, hipStream_t stream);
 int decode_plan(const qsdpa_decode_args* a, int* num_splits, int64_t* workspace_bytes, int64_t* ranges_bytes);

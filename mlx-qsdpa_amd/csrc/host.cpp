@@ -21,6 +21,7 @@
 #include <ATen/ATen.h>
 #include <ATen/TensorSubclassLikeUtils.h>
 #include <c10/core/GradMode.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
@@ -280,6 +281,54 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// The values of a plain CPU int64 vector; false for anything else.
+bool positions(PyObject* o, std::vector<int64_t>& x) {
+  if (!THPVariable_CheckExact(o)) return false;
+  const at::Tensor& t = THPVariable_Unpack(o);
+  if (!t.device().is_cpu() || t.layout() != at::kStrided || at::isTensorSubclassLike(t) || t.dim() != 1 ||
+      t.scalar_type() != at::kLong)
+    return false;
+  x.resize(t.numel());
+  for (int64_t i = 0; i < t.numel(); ++i) x[i] = t.data_ptr<int64_t>()[i * t.stride(0)];
+  return true;
+}
+
+// causal_mask(N, start, pad, window, device, stream): the bool mask
+// [B, 1, N, max(start) + N] for CPU vectors start and pad (or None), or
+// [N, start + N] for an int start and no pad, on GPU `device`; the negative
+// code of qsdpa_causal_mask; or None.
+PyObject* causal_mask(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  HANDLE_TH_ERRORS
+  int64_t N, first, window = int64_t(1) << 34, device, stream;
+  if (n != 6 || !as_int(a[0], N) || !as_int(a[4], device) || !as_int(a[5], stream) ||
+      (a[3] != Py_None && !as_int(a[3], window)) || c10::impl::dispatch_mode_enabled())
+    Py_RETURN_NONE;
+  int current = -1;
+  if (hipGetDevice(&current) != hipSuccess || current != device) Py_RETURN_NONE;
+  std::vector<int64_t> start, pad;
+  const bool one = as_int(a[1], first);
+  if (one) start.assign(1, first);
+  else if (!positions(a[1], start)) Py_RETURN_NONE;
+  if (a[2] != Py_None && (one || !positions(a[2], pad) || pad.size() != start.size())) Py_RETURN_NONE;
+  if (start.empty() || N < 1 || window > (int64_t(1) << 34) || window < -(int64_t(1) << 34)) Py_RETURN_NONE;
+  for (const auto* v : {&start, &pad})
+    for (int64_t x : *v)
+      if (x < INT32_MIN || x > INT32_MAX) Py_RETURN_NONE;
+  const int64_t B = start.size(), total = *std::max_element(start.begin(), start.end()) + N;
+  if (total < 1 || !fits32({B, N, total})) Py_RETURN_NONE;
+  const auto options = at::TensorOptions().dtype(at::kBool).device(at::kCUDA, static_cast<c10::DeviceIndex>(device));
+  at::Tensor out = one ? at::empty({N, total}, options) : at::empty({B, 1, N, total}, options);
+  qsdpa_causal_mask_args x = {};
+  x.B = B; x.N = N; x.total = total;
+  x.window = window;
+  x.start = start.data();
+  x.pad = pad.empty() ? nullptr : pad.data();
+  x.out = static_cast<uint8_t*>(out.data_ptr());
+  const int rc = qsdpa_causal_mask(&x, stream_of(stream));
+  return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(std::move(out));
+  END_HANDLE_TH_ERRORS
+}
+
 // A tensor that no gradient, of either mode, is taken through.
 bool constant(const at::Tensor& t) {
   return !(c10::GradMode::is_enabled() && t.requires_grad()) && !t._fw_grad(0).defined();
@@ -347,6 +396,7 @@ PyMethodDef methods[] = {
     {"columns", fast<columns>(), METH_FASTCALL, nullptr},
     {"grown", fast<grown>(), METH_FASTCALL, nullptr},
     {"decode", fast<decode>(), METH_FASTCALL, nullptr},
+    {"causal_mask", fast<causal_mask>(), METH_FASTCALL, nullptr},
     {"rotate", fast<rotate>(), METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };

@@ -36,6 +36,7 @@ EXPORTED_SYMBOLS = (
     "qsdpa_dequantize",
     "qsdpa_requant_window",
     "qsdpa_move_rows",
+    "qsdpa_causal_mask",
     "qsdpa_rotate",
     "qsdpa_last_error",
     "qsdpa_abi_version",

@@ -32,10 +32,18 @@ from . import kernels
 def _create_causal_mask(N, offset, window_size=None, left_padding=None, device=None):
     """cache.py:15-43.  Batched offsets give a bool (B, 1, N, max(offset)+N).
 
-    With a GPU `device` the mask is computed there from the (B,) offsets and
-    left padding, which are the only host-to-device copy (pinned, no wait)."""
+    With a GPU `device` the mask is computed there, by one launch that takes
+    the (B,) offsets and left padding in its arguments; what that does not take
+    (positions past 2^31, empty masks) by torch, after a pinned copy of them."""
     on_gpu = device is not None and torch.device(device).type == "cuda"
-    if isinstance(offset, torch.Tensor) and offset.dim() > 0:
+    batched = isinstance(offset, torch.Tensor) and offset.dim() > 0
+    if on_gpu:
+        pad = left_padding.to("cpu", torch.int64) if batched and left_padding is not None else None
+        mask = kernels.causal_mask(N, offset.to("cpu", torch.int64) if batched else int(offset), pad, window_size,
+                                   device)
+        if mask is not None:
+            return mask
+    if batched:
         off = offset.to("cpu", torch.int64)
         total = int(off.max()) + N
         dev = device if on_gpu else None

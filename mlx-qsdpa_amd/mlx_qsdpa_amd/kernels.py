@@ -252,6 +252,22 @@ def rotate(q, k, start, theta):
     return out
 
 
+def causal_mask(N, start, pad, window, device):
+    """The bool mask of N causal queries on GPU `device` in one launch
+    (csrc/causal_mask.hip): [N, start + N] for an int start, [B, 1, N,
+    max(start) + N] for CPU vectors start and pad (or None).  None for what
+    it does not take."""
+    if torch.jit.is_tracing() or torch.compiler.is_compiling():
+        return None
+    device = torch.device(device)
+    if device.index is None:
+        device = torch.device("cuda", torch.cuda.current_device())
+    out = _host().causal_mask(N, start, pad, window, device.index, torch.cuda.current_stream(device).cuda_stream)
+    if type(out) is int:
+        _lib.check(out)
+    return out
+
+
 class RowMove(NamedTuple):
     """Fill token columns [dst_col, dst_col + tokens) of batch row `dst_row` of
     a (B, H, N, W) buffer, every head: the columns dst_col + [copy_begin,
