@@ -7,8 +7,9 @@
 // math library's powf, sinf and cosf, so the results are the same bits.
 //
 // A decode step is bound by its launches: the torch expression is two copies
-// of positions to the device and 38 launches for q and k (54 us of kernels in
-// a 434 us step of a 2048-wide layer, the rest host time between them).
+// of positions to the device and 38 launches for q and k: one layer's step
+// (2048 wide, 16 / 4 heads of 128, batch of 2, 4096 keys) 404.9 us, 131.0 with
+// this kernel.
 //
 // One workgroup per token: the angles are shared by all heads, so each is
 // computed once (one lane per angle) and read from the LDS by the heads of q

@@ -88,8 +88,8 @@ def _rope(x, positions, theta):
 
 def _rotated(q, k, offset, theta):
     """q and k [B, H, L, D] at the positions offset (one, or one per
-    sequence) + l: one launch on the GPU, else the expression above.  At a
-    decode step of 2048-wide heads that took 40 launches and two copies."""
+    sequence) + l: one launch on the GPU, else the expression above (40
+    launches for the two, copies of the positions among them)."""
     if q.is_cuda and isinstance(theta, (int, float)):
         out = kernels.rotate(q, k, offset, float(theta))
         if out is not None:
