@@ -94,8 +94,11 @@ __global__ __launch_bounds__(256) void quantize_kernel(QuantJobs jobs) {
                                    p.db + off3(b, h, t, p.z_sb, p.z_sh, p.z_sn) + g);
 }
 
-// Jobs with at least this many groups take one lane per group.
-constexpr int64_t kWideJobGroups = 1 << 18;
+// Jobs with at least this many groups take GS / 32 lanes per group.  Whole
+// passes with GS / 8 against GS / 32 lanes: a 3000-token prompt (48000 groups
+// of 64, 4-bit) 132.1 against 130.7 us, 500 tokens onto 8 sequences (64000,
+// 8-bit) 175.4 against 173.2, a 1500-token prompt (12000) 42.55 against 43.1.
+constexpr int64_t kWideJobGroups = 1 << 15;
 
 template <typename Tag, int BITS, int GS, int L>
 void launch_quantize_l(const QuantJobs& j, bool vec, int64_t groups, int count, hipStream_t stream) {
