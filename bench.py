@@ -795,7 +795,7 @@ def main(argv=None) -> int:
         "whole_step": {"us": round(step_us, 3), "us_p5_p50_p95": _pcts(step_ms),
                        "what": "decode kernel + split-K merge, torch events on the launch stream"},
         "api_path": {"us_per_step": round(api_us, 3),
-                     "call": "mlx_qsdpa_amd.quantized_sdpa per step (argument block cached per geometry)"},
+                     "call": "mlx_qsdpa_amd.quantized_sdpa per step (native host path)"},
         "roofline": {
             "bound": "hbm",
             "achieved": round(kern_gbps, 1),
