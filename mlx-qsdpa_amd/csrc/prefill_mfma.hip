@@ -506,9 +506,16 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
   const int n_end = p.causal ? min(p.N, max(0, p.N - p.qL + (v_first + nrows - 1) / p.G + 1)) : p.N;
   const int len = max(n_end - s0, 0);
   constexpr int kTile = PG::Tile, NT = PG::NT, NU = PG::NU, KS = PG::KS;
-  int T_all = (len + kTile - 1) / kTile, j_first = 0;
+  // This split's tiles: [s_base, s_base + s_tiles) of the group's.
+  const int T_all = (len + kTile - 1) / kTile;
+  const int s_base = static_cast<int>(static_cast<int64_t>(split) * T_all / S);
+  const int s_tiles = static_cast<int>(static_cast<int64_t>(split + 1) * T_all / S) - s_base;
+  // [j_base, j_base + T): those of them that the mask leaves (the cut itself
+  // does not follow the mask: split partials round, so moving it would move
+  // the output).
+  int j_base = s_base, T = s_tiles;
   if constexpr (MASK) {
-    if (p.ranges) {  // [j_first, j_first + T_all): the tiles that the mask leaves
+    if (p.ranges) {
       const int2* rg = p.ranges + (static_cast<int64_t>(b) * groups_per_head + grp) * p.range_chunks;
       const int2 x = lane < p.range_chunks ? rg[lane] : int2{0, 0};
       const uint64_t m = __builtin_amdgcn_ballot_w64(x.y > 0);
@@ -517,13 +524,10 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
         lo = __builtin_amdgcn_readlane(x.x, static_cast<int>(__builtin_ctzll(m)));
         hi = __builtin_amdgcn_readlane(x.y, 63 - static_cast<int>(__builtin_clzll(m)));
       }
-      j_first = max(lo - s0, 0) / kTile;
-      T_all = max(min(T_all, (max(hi - s0, 0) + kTile - 1) / kTile) - j_first, 0);
+      j_base = max(s_base, max(lo - s0, 0) / kTile);
+      T = max(min(s_base + s_tiles, (max(hi - s0, 0) + kTile - 1) / kTile) - j_base, 0);
     }
   }
-  // This split's tiles: [j_base, j_base + T) of the group's.
-  const int j_base = j_first + static_cast<int>(static_cast<int64_t>(split) * T_all / S);
-  const int T = j_first + static_cast<int>(static_cast<int64_t>(split + 1) * T_all / S) - j_base;
 
   // The lane's row: v = v_first + 16 wave + r (clamped to the last real row).
   int n_lane, n_wave;  // the lane's key limit; the wave's smallest

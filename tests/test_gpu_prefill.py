@@ -429,3 +429,23 @@ def test_prefill_skips_masked_tiles(device, D, bits, gs, dtype, B, Hq, Hkv, N, L
     _check(q, kq, vq, bits, gs, "per head", mask=heads)
     _check(q, kq, vq, bits, gs, "nothing", mask=torch.zeros_like(keep))
     _check(q, kq, vq, bits, gs, "everything", mask=torch.ones_like(keep), causal=True)
+
+
+@pytest.mark.parametrize("D,bits,gs,dtype", [(128, 4, 64, torch.float16), (128, 8, 128, torch.bfloat16),
+                                             (256, 4, 32, torch.float16), (64, 8, 64, torch.bfloat16)])
+@pytest.mark.parametrize("B,Hq,Hkv,N,L", [(3, 32, 8, 1001, 333), (1, 16, 2, 4099, 130)], ids=["rounds", "splits"])
+def test_prefill_mask_shared_by_the_heads_gives_the_bits_of_one_each(device, D, bits, gs, dtype, B, Hq, Hkv, N, L):
+    """A mask of one row set for all heads leaves out tiles, one per head does
+    not: the outputs are the same bits, in one pass and with key splits (whose
+    cut, and so their partials' rounding, must not follow the mask)."""
+    if D == 64:
+        Hq = Hkv * 8
+    q, kq, vq = _inputs(B, Hq, Hkv, N, L, bits, gs, dtype, seed=N + 1, D=D)
+    keep = _block_mask(B, L, N, seed=L + 1).to(device)
+    print(f"prefill shared mask D={D} {dtype} N={N} L={L}", flush=True)
+    call = dict(scale=D ** -0.5, bits=bits, group_size=gs)
+    args = (q, kq[0], vq[0], kq[1], vq[1], kq[2], vq[2])
+    shared = kernels.decode(*args, mask=keep, **call)
+    each = kernels.decode(*args, mask=keep.expand(B, Hq, L, N).contiguous(), **call)
+    torch.cuda.synchronize()
+    assert torch.equal(shared, each)
