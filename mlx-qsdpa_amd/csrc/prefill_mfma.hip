@@ -50,11 +50,11 @@
 // exactly as mx.dequantize rounds it, then scaled by 2^-k and converted to
 // float16, which is exact for magnitudes from 2^-17 up (below that the error
 // is at most 2^-25 * 2^k).  A scan of the workgroup's V scales and biases
-// gives max |V| (at code 0 or 2^bits - 1 of each group): k is 0 unless it
-// reaches kVBound (the output is scaled back by 2^k), and P (in [0, 256])
-// enters as one float16 term -- the float16 path's 11 significant bits, one
-// MFMA per block -- while max |V| is at most kPVSingle, as two terms (hi +
-// lo, 22 bits) above it.
+// gives max |V| (at code 0 or 2^bits - 1 of each group): k is 0 unless that
+// of the staged keys reaches kVBound (the output is scaled back by 2^k), and
+// P (in [0, 256]) enters as one float16 term -- the float16 path's 11
+// significant bits, one MFMA per block -- while that of the keys within the
+// limit is at most kPVSingle, as two terms (hi + lo, 22 bits) above it.
 //
 // Rows of a kv head are (position v / G, head v % G) as in the decode
 // kernel; a causal mask (aligned to the last key), kv_start (keys before it
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
   using PG = PGeo<D>;
   using P = Prefill<Tag, D, BITS, GS>;
   __shared__ __attribute__((aligned(16))) uint8_t s_buf[4 * PG::BufBytes];
-  __shared__ float s_red[kPWaves];
+  __shared__ float s_red[2][kPWaves];
 
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -761,17 +761,19 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
     P::load(R1, src, row_of(1));
     bool two = false;
     if constexpr (Tag::kId == QSDPA_BF16) {
-      // max |V| of this workgroup's keys: a group's values are affine in
-      // the code, so its largest magnitude is at code 0 or 2^bits - 1.  To
-      // the end of the last tile: keys past the causal limit are staged with
-      // it, and P = 0 does not cancel one that float16 cannot hold.
+      // max |V| of the keys: a group's values are affine in the code, so its
+      // largest magnitude is at code 0 or 2^bits - 1.  `bound`: of the
+      // split's keys within the limit, which chooses P's terms (keys that no
+      // row sees must not move an output, nor a mask the choice).  `staged`:
+      // to the end of the last tile, whose keys past the causal limit are
+      // staged with it: P = 0 does not cancel one that float16 cannot hold.
       constexpr int NG = D / GS;
       constexpr float kCodeMax = static_cast<float>((1 << BITS) - 1);
       // Eight rows per thread in flight (rows past the range read the
       // range's first row again: no effect on the maximum).
       constexpr int kRows = 8;
-      float bound = 0.0f;
-      const int t_lo = j_base * kTile, t_hi = min((j_base + T) * kTile, p.N - s0);
+      float bound = 0.0f, staged = 0.0f;
+      const int t_lo = s_base * kTile, t_hi = min((s_base + s_tiles) * kTile, p.N - s0);
       for (int t0 = t_lo + tid; t0 < t_hi; t0 += kRows * kPThreads) {
         uint16_t sv[kRows][NG], bv[kRows][NG];
 #pragma unroll
@@ -784,27 +786,40 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
           }
         }
 #pragma unroll
-        for (int u = 0; u < kRows; ++u)
+        for (int u = 0; u < kRows; ++u) {
+          float x = 0.0f;
 #pragma unroll
           for (int g = 0; g < NG; ++g) {
             const float s = bf16_bits_to_f32(sv[u][g]), b = bf16_bits_to_f32(bv[u][g]);
-            bound = fmaxf(bound, fmaxf(fabsf(b), fabsf(fmaf(s, kCodeMax, b))));
+            x = fmaxf(x, fmaxf(fabsf(b), fabsf(fmaf(s, kCodeMax, b))));
           }
+          staged = fmaxf(staged, x);
+          if (t0 + u * kPThreads < len) bound = fmaxf(bound, x);
+        }
       }
 #pragma unroll
-      for (int o = 1; o < 64; o <<= 1) bound = fmaxf(bound, shfl_xor_f32(bound, o));
-      if (lane == 0) s_red[wave] = bound;
+      for (int o = 1; o < 64; o <<= 1) {
+        bound = fmaxf(bound, shfl_xor_f32(bound, o));
+        staged = fmaxf(staged, shfl_xor_f32(staged, o));
+      }
+      if (lane == 0) {
+        s_red[0][wave] = bound;
+        s_red[1][wave] = staged;
+      }
       __syncthreads();
 #pragma unroll
-      for (int i = 0; i < kPWaves; ++i) bound = fmaxf(bound, s_red[i]);
+      for (int i = 0; i < kPWaves; ++i) {
+        bound = fmaxf(bound, s_red[0][i]);
+        staged = fmaxf(staged, s_red[1][i]);
+      }
       two = !(bound <= kPVSingle);
-      if (bound > kVBound || D == 64) {
-        // k = 1 + floor(log2(bound / kVBound)), so that bound 2^-k < kVBound.
-        // A finite bfloat16 bound (< 2^128) needs k <= 113; the clamp keeps
+      if (staged > kVBound || D == 64) {
+        // k = 1 + floor(log2(staged / kVBound)), so that staged 2^-k < kVBound.
+        // A finite bfloat16 value (< 2^128) needs k <= 113; the clamp keeps
         // k <= 126 when the scan overflowed to Inf, so that 2^-k and 2^k
         // stay normal floats.  D = 64: also up (k < 0), at least to k = -100,
         // where 2^-k 2^24 is still finite.
-        const float x = fminf(D == 64 ? fmaxf(bound * (1.0f / kVBound), 0x1p-101f) : bound * (1.0f / kVBound), 0x1p125f);
+        const float x = fminf(D == 64 ? fmaxf(staged * (1.0f / kVBound), 0x1p-101f) : staged * (1.0f / kVBound), 0x1p125f);
         const int k = static_cast<int>((__builtin_bit_cast(uint32_t, x) >> 23) & 0xFFu) - 126;
         vsc = __builtin_bit_cast(float, static_cast<uint32_t>(127 - k) << 23);
         osc = __builtin_bit_cast(float, static_cast<uint32_t>(127 + k) << 23);

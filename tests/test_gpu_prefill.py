@@ -449,3 +449,28 @@ def test_prefill_mask_shared_by_the_heads_gives_the_bits_of_one_each(device, D, 
     each = kernels.decode(*args, mask=keep.expand(B, Hq, L, N).contiguous(), **call)
     torch.cuda.synchronize()
     assert torch.equal(shared, each)
+
+
+@pytest.mark.parametrize("bits,gs", [(4, 64), (8, 128)])
+def test_prefill_keys_past_the_limit_leave_the_bits_alone(device, bits, gs):
+    """bfloat16 P enters P.V in one term or two by max |V| of the keys that
+    the row group sees: larger values past the causal limit, in the group's
+    last tile, do not change the bits of its rows."""
+    Hq, Hkv, L = 6, 2, 300
+    group = 128 // (Hq // Hkv)  # whole positions of the first row group: keys [0, 43), a tile to 64
+    q, kq, vq = _inputs(1, Hq, Hkv, L, L, bits, gs, torch.bfloat16, seed=9)
+    vq = (vq[0], *((t.float() * 0.5).to(torch.bfloat16) for t in vq[1:]))  # below the bound of one term
+    assert float(to.dequantize(*vq, gs, bits, torch.bfloat16).abs().max()) < 8
+    print(f"prefill past the limit bits={bits}", flush=True)
+
+    def run():
+        return kernels.decode(q, kq[0], vq[0], kq[1], vq[1], kq[2], vq[2], scale=128 ** -0.5, bits=bits,
+                              group_size=gs, causal=True)
+
+    want = run()
+    for t in vq[1:]:
+        t[:, :, group + 1:] *= 100
+    got = run()
+    torch.cuda.synchronize()
+    assert torch.equal(got[:, :, :group], want[:, :, :group])
+    assert not torch.equal(got[:, :, group + 1:], want[:, :, group + 1:])
