@@ -182,9 +182,10 @@ int qsdpa_decode(const qsdpa_decode_args* args, void* stream);
  * QSDPA_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends.
  * Arguments whose partials need more (qsdpa_decode_workspace_size) return
  * QSDPA_ERR_WORKSPACE.  The call allocates and frees nothing (the first
- * call on a device looks the array's address up).  Every call on one GPU
- * shares that GPU's array: calls that overlap on one GPU (two streams, two
- * host threads) race and must be serialised by the caller.
+ * call on a device looks the array's address up).  Every split-K call on one
+ * GPU shares that GPU's array: such calls that overlap on one GPU (two
+ * streams, two host threads) race and must be serialised by the caller.  A
+ * single pass (num_splits 1) does not touch the array.
  */
 #define QSDPA_NOALLOC_SCRATCH_BYTES (16u << 20)
 int qsdpa_decode_noalloc(const qsdpa_decode_args* args, void* stream);

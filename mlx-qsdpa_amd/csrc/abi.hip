@@ -386,11 +386,9 @@ int qsdpa_decode_noalloc(const qsdpa_decode_args* args, void* stream) {
   int64_t ws = 0, extra = 0;
   rc = decode_plan(args, &splits, &ws, &extra);
   if (rc) return rc;
-  void *scratch_ptr = nullptr, *ranges = nullptr;
-  if (extra > 0 && ranges_at(ws) + extra <= static_cast<int64_t>(kScratchBytes)) {
-    if ((rc = scratch_address(&scratch_ptr))) return rc;
-    ranges = static_cast<uint8_t*>(scratch_ptr) + ranges_at(ws);
-  }
+  // No key ranges here: a single pass leaves the shared array alone, so such
+  // calls may overlap on one GPU.
+  void* scratch_ptr = nullptr;
   if (splits > 1) {
     if (ws > static_cast<int64_t>(kScratchBytes))
       return fail(QSDPA_ERR_WORKSPACE,
@@ -399,7 +397,7 @@ int qsdpa_decode_noalloc(const qsdpa_decode_args* args, void* stream) {
                   static_cast<long long>(ws), static_cast<long long>(kScratchBytes));
     if ((rc = scratch_address(&scratch_ptr))) return rc;
   }
-  return run_decode(args, splits, scratch_ptr, ranges, static_cast<hipStream_t>(stream));
+  return run_decode(args, splits, scratch_ptr, nullptr, static_cast<hipStream_t>(stream));
 }
 
 int qsdpa_quantize(const qsdpa_quantize_args* a, void* stream) {

@@ -143,3 +143,33 @@ def test_noalloc_refuses_partials_beyond_the_scratch(device):
     assert rc == _lib.QSDPA_ERR_WORKSPACE
     assert b"static scratch" in lib.qsdpa_last_error()
     del keep
+
+
+def _graph_nodes(launch):
+    """Launches that `launch(stream)` records under capture (nothing runs)."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        launch(torch.cuda.current_stream().cuda_stream)
+    n = ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(ctypes.c_void_p(graph.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+    return n.value
+
+
+def test_noalloc_single_pass_leaves_the_scratch_alone(device):
+    """A masked prefill in one pass is the prefill kernel alone: calls that
+    overlap on one GPU share nothing (a workspace's key ranges would be a
+    launch of their own that writes the shared array)."""
+    lib = _lib.load()
+    B, Hq, Hkv, N, qL, D, bits, gs = 3, 32, 8, 700, 333, 128, 4, 64
+    q = torch.zeros((B, Hq, qL, D), dtype=torch.float16, device=device)
+    kp = torch.zeros((B, Hkv, N, D * bits // 32), dtype=torch.uint32, device=device)
+    sc = torch.zeros((B, Hkv, N, D // gs), dtype=torch.float16, device=device)
+    mask = torch.ones((B, 1, qL, N), dtype=torch.bool, device=device)
+    out = torch.zeros_like(q)
+    a, keep = kernels._decode_args(q, kp, kp, sc, sc, sc, sc, out, 1.0, bits, gs, mask, None, 0)
+    n = ctypes.c_int32(0)
+    _lib.check(lib.qsdpa_decode_workspace_size(ctypes.byref(a), ctypes.byref(n)))
+    assert n.value == 1
+    assert _graph_nodes(lambda s: _lib.check(lib.qsdpa_decode_noalloc(ctypes.byref(a), s))) == 1
+    del keep
