@@ -49,7 +49,7 @@
 extern "C" {
 #endif
 
-#define QSDPA_ABI_VERSION 6
+#define QSDPA_ABI_VERSION 7
 
 enum {
   QSDPA_OK = 0,
@@ -164,14 +164,25 @@ typedef struct {
 } qsdpa_decode_args;
 
 /* Bytes of workspace qsdpa_decode needs for these args (0 for a single
- * pass), and for a prefill under a mask the bytes that let it leave out the
- * key tiles that the mask rules out (with less it reads every tile).  If num_splits_out is not NULL it receives the split count that
+ * pass).  If num_splits_out is not NULL it receives the split count that
  * qsdpa_decode will use.  Returns a negative QSDPA_ERR_* on bad args.     */
 int64_t qsdpa_decode_workspace_size(const qsdpa_decode_args* args,
                                     int32_t* num_splits_out);
 
 /* Launch the decode on `stream`. */
 int qsdpa_decode(const qsdpa_decode_args* args, void* stream);
+
+/*
+ * qsdpa_decode with a buffer in which a prefill under a mask notes the keys
+ * that the mask leaves each group of its rows, to leave out the tiles without
+ * any (the same results, to the bit).  qsdpa_decode_range_bytes: the bytes
+ * that such a call has use for, 0 for the others (or a negative QSDPA_ERR_*).
+ * ranges: device memory, 16-byte aligned, of any contents, written by the
+ * call: calls that overlap in time need buffers of their own.  With NULL or
+ * fewer bytes the call is qsdpa_decode, which reads every tile.
+ */
+int64_t qsdpa_decode_range_bytes(const qsdpa_decode_args* args);
+int qsdpa_decode_ranges(const qsdpa_decode_args* args, void* ranges, int64_t ranges_bytes, void* stream);
 
 /*
  * qsdpa_decode without a caller workspace: no counterpart in the reference.

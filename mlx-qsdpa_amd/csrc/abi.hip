@@ -231,7 +231,7 @@ bool fused_merge(const qsdpa_decode_args* a, int splits, bool prefill, bool mfma
 // than 64 keys per split, and no more than kMaxSplits.
 //
 // *workspace_bytes: what the call must have; *ranges_bytes: what it has use
-// for beyond that (a prefill's key ranges under its mask), at the end.
+// for beyond that (a prefill's key ranges under its mask).
 int decode_plan(const qsdpa_decode_args* a, int* num_splits, int64_t* workspace_bytes, int64_t* ranges_bytes) {
   // Many query positions per kv head: the prefill kernel, with key splits
   // where its row groups alone would leave CUs idle.
@@ -260,10 +260,6 @@ int decode_plan(const qsdpa_decode_args* a, int* num_splits, int64_t* workspace_
   *ranges_bytes = prefill ? prefill_range_bytes(a) : 0;
   return QSDPA_OK;
 }
-
-// Where a call's key ranges lie in its workspace: behind what the call must
-// have, and in a single pass behind the counters, which stay zero.
-int64_t ranges_at(int64_t workspace_bytes) { return std::max(workspace_bytes, kTicketBytes); }
 
 // Launch the decode for validated arguments: the main kernel, then (split-K)
 // the merge, with the partials in `workspace` (decode_plan's layout).
@@ -353,10 +349,20 @@ int64_t qsdpa_decode_workspace_size(const qsdpa_decode_args* args, int32_t* num_
   rc = decode_plan(args, &splits, &ws, &extra);
   if (rc) return rc;
   if (num_splits_out) *num_splits_out = splits;
-  return extra > 0 ? ranges_at(ws) + extra : ws;
+  return ws;
 }
 
-int qsdpa_decode(const qsdpa_decode_args* args, void* stream) {
+int64_t qsdpa_decode_range_bytes(const qsdpa_decode_args* args) {
+  clear_error();
+  int rc = validate_decode(args);
+  if (rc) return rc;
+  int splits = 1;
+  int64_t ws = 0, extra = 0;
+  rc = decode_plan(args, &splits, &ws, &extra);
+  return rc ? rc : extra;
+}
+
+int qsdpa_decode_ranges(const qsdpa_decode_args* args, void* ranges, int64_t ranges_bytes, void* stream) {
   clear_error();
   int rc = validate_decode(args);
   if (rc) return rc;
@@ -370,13 +376,12 @@ int qsdpa_decode(const qsdpa_decode_args* args, void* stream) {
                   static_cast<long long>(ws), static_cast<long long>(args->workspace_bytes));
     if (!aligned(args->workspace, 16)) return fail(QSDPA_ERR_INVALID, "workspace not 16-byte aligned");
   }
-  // A prefill whose workspace ends before the key ranges takes its mask as it is.
-  void* ranges = nullptr;
-  if (extra > 0 && args->workspace && static_cast<int64_t>(args->workspace_bytes) >= ranges_at(ws) + extra &&
-      aligned(args->workspace, 16))
-    ranges = static_cast<uint8_t*>(args->workspace) + ranges_at(ws);
+  if (extra == 0 || ranges_bytes < extra) ranges = nullptr;
+  if (ranges && !aligned(ranges, 16)) return fail(QSDPA_ERR_INVALID, "ranges not 16-byte aligned");
   return run_decode(args, splits, args->workspace, ranges, static_cast<hipStream_t>(stream));
 }
+
+int qsdpa_decode(const qsdpa_decode_args* args, void* stream) { return qsdpa_decode_ranges(args, nullptr, 0, stream); }
 
 int qsdpa_decode_noalloc(const qsdpa_decode_args* args, void* stream) {
   clear_error();

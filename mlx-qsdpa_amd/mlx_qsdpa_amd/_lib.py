@@ -23,13 +23,15 @@ QSDPA_BF16 = 1
 QSDPA_F32 = 2
 QSDPA_BOOL = 3
 
-ABI_VERSION = 6
+ABI_VERSION = 7
 NOALLOC_SCRATCH_BYTES = 16 << 20
 
 # Every symbol include/qsdpa.h declares.
 EXPORTED_SYMBOLS = (
     "qsdpa_decode_workspace_size",
     "qsdpa_decode",
+    "qsdpa_decode_range_bytes",
+    "qsdpa_decode_ranges",
     "qsdpa_decode_noalloc",
     "qsdpa_quantize",
     "qsdpa_quantize_batch",
@@ -132,11 +134,22 @@ def load(path: os.PathLike | str | None = None) -> ctypes.CDLL:
             f"{p} is missing: build it with `python mlx-qsdpa_amd/build_lib.py` "
             "(the quantized SDPA path has no non-HIP fallback)")
     lib = ctypes.CDLL(str(p))
+    lib.qsdpa_abi_version.argtypes = []
+    lib.qsdpa_abi_version.restype = ctypes.c_int
+    ver = lib.qsdpa_abi_version()
+    if ver != ABI_VERSION:
+        raise ImportError(f"{p}: ABI version {ver}, expected {ABI_VERSION}: build it again with "
+                          "`python mlx-qsdpa_amd/build_lib.py`")
     lib.qsdpa_decode_workspace_size.argtypes = [ctypes.POINTER(DecodeArgs),
                                                 ctypes.POINTER(ctypes.c_int32)]
     lib.qsdpa_decode_workspace_size.restype = ctypes.c_int64
     lib.qsdpa_decode.argtypes = [ctypes.POINTER(DecodeArgs), ctypes.c_void_p]
     lib.qsdpa_decode.restype = ctypes.c_int
+    lib.qsdpa_decode_range_bytes.argtypes = [ctypes.POINTER(DecodeArgs)]
+    lib.qsdpa_decode_range_bytes.restype = ctypes.c_int64
+    lib.qsdpa_decode_ranges.argtypes = [ctypes.POINTER(DecodeArgs), ctypes.c_void_p, ctypes.c_int64,
+                                        ctypes.c_void_p]
+    lib.qsdpa_decode_ranges.restype = ctypes.c_int
     lib.qsdpa_decode_noalloc.argtypes = [ctypes.POINTER(DecodeArgs), ctypes.c_void_p]
     lib.qsdpa_decode_noalloc.restype = ctypes.c_int
     lib.qsdpa_quantize.argtypes = [ctypes.POINTER(QuantizeArgs), ctypes.c_void_p]
@@ -151,11 +164,6 @@ def load(path: os.PathLike | str | None = None) -> ctypes.CDLL:
     lib.qsdpa_move_rows.restype = ctypes.c_int
     lib.qsdpa_last_error.argtypes = []
     lib.qsdpa_last_error.restype = ctypes.c_char_p
-    lib.qsdpa_abi_version.argtypes = []
-    lib.qsdpa_abi_version.restype = ctypes.c_int
-    ver = lib.qsdpa_abi_version()
-    if ver != ABI_VERSION:
-        raise ImportError(f"{p}: ABI version {ver}, expected {ABI_VERSION}")
     if path is None:
         _lib = lib
     return lib

@@ -473,13 +473,16 @@ class DecodePlan:
         ws = _lib.check(self.lib.qsdpa_decode_workspace_size(ctypes.byref(self.args),
                                                              ctypes.byref(n)))
         self.num_splits = int(n.value)
-        self.workspace = None
+        self.workspace = self._ranges = None
         if ws > 0:
             # Zero-filled: the split merge's counters at its start must be
             # zero before the first call (each call leaves them zero).
             self.workspace = torch.zeros(ws, dtype=torch.uint8, device=q.device)
             self.args.workspace = self.workspace.data_ptr()
             self.args.workspace_bytes = ws
+        if mask is not None:
+            n = _lib.check(self.lib.qsdpa_decode_range_bytes(ctypes.byref(self.args)))
+            self._ranges = torch.empty(n, dtype=torch.uint8, device=q.device) if n > 0 else None
         self._args_ref = ctypes.byref(self.args)
         self.device = q.device
         self.args.num_splits = self.num_splits  # fixed from here on (set_keys)
@@ -496,7 +499,11 @@ class DecodePlan:
             self.args.prof_begin, self.args.prof_end = prof_events
         else:
             self.args.prof_begin = self.args.prof_end = None
-        _lib.check(self.lib.qsdpa_decode(self._args_ref, _stream(self.q)))
+        r = self._ranges
+        if r is None:
+            _lib.check(self.lib.qsdpa_decode(self._args_ref, _stream(self.q)))
+        else:
+            _lib.check(self.lib.qsdpa_decode_ranges(self._args_ref, r.data_ptr(), r.numel(), _stream(self.q)))
         return self.out
 
 
@@ -598,16 +605,25 @@ def decode(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size, mask=None, kv_
     lib = _lib.load()
     n = ctypes.c_int32(0)
     ws = _lib.check(lib.qsdpa_decode_workspace_size(ctypes.byref(a), ctypes.byref(n)))
+    # A masked prefill's key ranges lie behind the counters and the partials.
+    rb = _lib.check(lib.qsdpa_decode_range_bytes(ctypes.byref(a))) if mask is not None and q.shape[2] > 1 else 0
+    at = max(ws, _TICKET_BYTES)
+    given = workspace is not None and workspace.numel() >= ws
+    ranges = None
+    if rb > 0 or (ws > 0 and not given):
+        total = at + rb if rb > 0 else ws
+        held = _capture_workspace(q.device, total) if torch.cuda.is_current_stream_capturing() \
+            else _workspace(q.device, _stream(q), total)
+        ranges = held.data_ptr() + at
+        if not given:
+            workspace = held
     if ws > 0:
-        if workspace is None or workspace.numel() < ws:
-            if torch.cuda.is_current_stream_capturing():
-                workspace = _capture_workspace(q.device, ws)
-            else:
-                workspace = _workspace(q.device, _stream(q), ws)
-        a.workspace = workspace.data_ptr()
-        a.workspace_bytes = ws
+        a.workspace, a.workspace_bytes = workspace.data_ptr(), ws
     if prof_events is not None:
         a.prof_begin, a.prof_end = prof_events
-    _lib.check(lib.qsdpa_decode(ctypes.byref(a), _stream(q)))
+    if rb > 0:
+        _lib.check(lib.qsdpa_decode_ranges(ctypes.byref(a), ranges, rb, _stream(q)))
+    else:
+        _lib.check(lib.qsdpa_decode(ctypes.byref(a), _stream(q)))
     del keep_alive
     return out

@@ -272,3 +272,35 @@ int main() {{
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", str(src), "-o", str(exe)], check=True)
     out = subprocess.run([str(exe)], capture_output=True, text=True)
     assert out.returncode == 0 and out.stdout.strip() == "ok", out.stdout
+
+
+def _masked_prefill(B, Hq, Hkv, N, L, D=128, bits=8, gs=128, mask=None):
+    """Arguments of a prefill under a bool mask (stand-in addresses, never
+    dereferenced); mask: (stride_b, stride_h, stride_n, stride_q)."""
+    a = _lib.DecodeArgs()
+    a.B, a.H_q, a.H_kv, a.N, a.D = B, Hq, Hkv, N, D
+    a.bits, a.group_size, a.dtype, a.scale, a.q_len = bits, gs, _lib.QSDPA_BF16, 0.1, L
+    W, G, base = D * bits // 32, D // gs, 1 << 20
+    a.q = a.out = _lib.View(base, Hq * L * D, L * D, D)
+    a.k_packed = a.v_packed = _lib.View(base, Hkv * N * W, N * W, W)
+    a.k_scales = a.v_scales = a.k_biases = a.v_biases = _lib.View(base, Hkv * N * G, N * G, G)
+    sb, sh, sn, sq = mask or (L * N, 0, 1, N)
+    a.mask, a.mask_dtype, a.mask_stride_q = _lib.View(base, sb, sh, sn), _lib.QSDPA_BOOL, sq
+    return a
+
+
+def test_a_single_masked_pass_needs_no_workspace():
+    """The key ranges of a masked prefill are a buffer of their own, which
+    the caller may leave out: a workspace is split-K's alone, and a single
+    pass neither needs one nor writes one that it is given."""
+    lib = _lib.load()
+    n = ctypes.c_int32(0)
+    a = _masked_prefill(8, 32, 8, 1500, 500)
+    assert lib.qsdpa_decode_workspace_size(ctypes.byref(a), ctypes.byref(n)) == 0 and n.value == 1
+    assert lib.qsdpa_decode_range_bytes(ctypes.byref(a)) >= 8 * 16 * 2 * 8  # 16 row groups, 2 chunks of 1024 keys
+    for mask in ((1500 * 500 * 32, 1500 * 500, 1, 1500), (3000 * 500, 0, 2, 3000)):  # per head; every other byte
+        assert lib.qsdpa_decode_range_bytes(ctypes.byref(_masked_prefill(8, 32, 8, 1500, 500, mask=mask))) == 0
+    a.mask.ptr = None
+    assert lib.qsdpa_decode_range_bytes(ctypes.byref(a)) == 0
+    a.bits = 3
+    assert lib.qsdpa_decode_range_bytes(ctypes.byref(a)) == _lib.QSDPA_ERR_INVALID
