@@ -45,7 +45,7 @@ int launch_decode_mfma(const qsdpa_decode_args* a, int num_splits, float* part_a
 // Defined in prefill_mfma.hip.
 bool prefill_supports(const qsdpa_decode_args* a);
 int prefill_num_splits(const qsdpa_decode_args* a, int cus);
-int64_t prefill_range_bytes(const qsdpa_decode_args* a);
+int64_t prefill_range_bytes(const qsdpa_decode_args* a, int splits, int cus);
 int launch_prefill_mfma(const qsdpa_decode_args* a, int splits, float* part_acc, float* part_ml, void* ranges,
                         hipStream_t stream);
 // Defined in decode_rows32.hip (rows32_supports: abi_internal.h).
@@ -257,7 +257,7 @@ int decode_plan(const qsdpa_decode_args* a, int* num_splits, int64_t* workspace_
   // (U + B, U = splits * B) under the stream-K schedule of a left-padded
   // batch; then that schedule's (first column, count) per sequence.
   *workspace_bytes = splits > 1 ? workspace_layout(a, splits).total : 0;
-  *ranges_bytes = prefill ? prefill_range_bytes(a) : 0;
+  *ranges_bytes = prefill ? prefill_range_bytes(a, splits, compute_units()) : 0;
   return QSDPA_OK;
 }
 

@@ -352,14 +352,16 @@ struct Prefill {
 // mask once, and a row group then runs from the tile of its first attended
 // key to that of its last.  Only masks whose keys are adjacent and whose rows
 // are shared by the heads: one pass over one head's mask then serves all of
-// them.  Memory-latency bound; 2.5 us for 8 masks of 500 x 1500 bools.
+// them.  Memory-latency bound; 7.6 us traced for 8 masks of 500 x 1500 bools, a
+// launch included.
 //
-// At that chunk (8 sequences of 32 / 8 heads, 8-bit bf16; attention alone)
-// 137.5 us under the batch cache's mask against 200 over every tile, 193 under
-// one causal mask for all.  The same look inside the prefill kernel, by each
-// workgroup for itself, took 176, a list there of the tiles with an attended
-// key 164 (and 249 instead of 200 for a mask with holes everywhere: an index
-// from the LDS per tile).
+// What it is worth (that chunk, 32 / 8 heads, 8-bit bf16, the call): 172 us
+// under the batch cache's mask against 202 over every tile.  What it costs: a
+// mask that leaves no tile out (all true, or holes everywhere) takes 219
+// against 201.  Calls that cannot gain go without (prefill_range_bytes).  The
+// same look inside the prefill kernel, by each workgroup for itself, was 38 us
+// slower, a list there of the tiles with an attended key 27 us (and 42 us
+// slower for a mask with holes everywhere: an index from the LDS per tile).
 __host__ __device__ constexpr int mask_bytes(int kind) {
   return kind == QSDPA_BOOL ? 1 : kind == QSDPA_F32 ? 4 : 2;
 }
@@ -463,25 +465,27 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
   // robin, so the work of workgroup id w goes to XCD w % 8 in consecutive
   // runs: the row groups of one (batch, kv head) share one XCD's L2.
   //
-  // Causal calls (and those with a mask tensor, which mostly is causal too) of
-  // several rounds of workgroups: a row group's work grows with its position,
-  // so each head's groups run from the longest down (the last workgroups to
-  // start are then the shortest), and where the heads do not divide evenly
-  // over the XCDs the heads alternate instead, so that no XCD holds only long
-  // groups.  A prompt of 3000 tokens (32 / 8 heads, 4-bit; 752 workgroups),
-  // with its cache update: 142.6 us against 156.5 with the shortest groups
-  // first.  Where the sequences' key ranges may differ (a start each, or a
-  // mask), an XCD takes every eighth head, so that it does not hold one
-  // sequence alone: 8 sequences of 500 x 1500 (32 / 8 heads, 8-bit bf16) under
-  // the batch cache's mask 137.5 us against 195 in runs, with a start each and
-  // the causal limit 134 against 154; a mask with random holes everywhere,
-  // whose rows then pass through every XCD's L2, takes 218 against 207.
+  // Causal calls (and those whose mask's key ranges are known, which mostly is
+  // causal too) of several rounds of workgroups: a row group's work grows with
+  // its position, so each head's groups run from the longest down (the last
+  // workgroups to start are then the shortest), and where the heads do not
+  // divide evenly over the XCDs the heads alternate instead, so that no XCD
+  // holds only long groups.  A prompt of 3000 tokens (32 / 8 heads, 4-bit; 752
+  // workgroups), with its cache update: 142.6 us against 156.5 with the
+  // shortest groups first.  Where the sequences' key ranges may differ (a
+  // start each, or a mask's ranges), an XCD takes every eighth head, so that
+  // it does not hold one sequence alone: 8 sequences of 500 x 1500 (32 / 8
+  // heads, 8-bit bf16), kernel alone, under the batch cache's mask 182 us
+  // against 221 in runs (227 without the ranges); a mask with random holes
+  // everywhere 229 against 226 (221).  A mask without ranges keeps the runs:
+  // 2 sequences of 512 x 2048 in one round of 256 workgroups 64.1 against 66.0.
   const int total = gridDim.x;
   const int heads = p.Hkv * p.B;
   const int S = p.num_splits;
-  const bool uneven = p.B > 1 && (MASK || p.kv_start);
+  const bool ranged = MASK && p.ranges;
+  const bool uneven = p.B > 1 && ((ranged && p.m_sb != 0) || p.kv_start);
   int w = blockIdx.x, split = 0, grp, head;
-  if ((p.causal || MASK || uneven) && S == 1 && heads % 8 != 0) {
+  if ((p.causal || ranged || uneven) && S == 1 && heads % 8 != 0) {
     head = w % heads;
     grp = w / heads;
   } else if (uneven && S == 1) {
@@ -494,7 +498,7 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
     grp = w % groups_per_head;
     head = w / groups_per_head;
   }
-  if (p.causal || MASK) grp = groups_per_head - 1 - grp;
+  if (p.causal || ranged) grp = groups_per_head - 1 - grp;
   const int kvh = head % p.Hkv;
   const int b = head / p.Hkv;
 
@@ -1024,13 +1028,21 @@ int prefill_num_splits(const qsdpa_decode_args* a, int cus) {
   return static_cast<int>(std::max<int64_t>(s, 1));
 }
 
-// Workspace bytes of the row groups' key ranges under the call's mask; 0
-// where the kernel takes the mask as it is (heads with masks of their own,
-// keys that are not adjacent, more groups than a grid dimension holds).
-int64_t prefill_range_bytes(const qsdpa_decode_args* a) {
+// Bytes of the row groups' key ranges under the call's mask; 0 where the
+// kernel takes the mask as it is: heads with masks of their own, keys that
+// are not adjacent, more groups than a grid dimension holds, and calls whose
+// workgroups all run at once (one per CU: so every call with key splits too),
+// which take as long as their longest group whatever the others leave out.
+// With the ranges such calls lost their launch: a batch of 2, 32 / 8 heads,
+// 512 x 2048, 4-bit (256 workgroups) 69.2 us under a left-padded mask against
+// 59.4, 1024 x 4096 8-bit (256) 136.1 against 128.3, 64 x 3000 with splits
+// 43.4 against 35.4.  From 264 workgroups on they win where the mask leaves
+// tiles out (304 of 600 x 2000 at D = 256: 237 against 285).
+int64_t prefill_range_bytes(const qsdpa_decode_args* a, int splits, int cus) {
   if (!a->mask.ptr || a->mask.stride_n != 1 || a->mask.stride_h != 0) return 0;
   const int64_t groups = (static_cast<int64_t>(a->H_q / a->H_kv) * a->q_len + kPGroupRows - 1) / kPGroupRows;
   if (groups > 65535 || a->B > 65535) return 0;
+  if (splits > 1 || groups * a->H_kv * a->B <= cus) return 0;
   const int64_t chunks = (a->N + range_chunk(a->N) - 1) / range_chunk(a->N);
   return (groups * a->B * chunks * 8 + 255) / 256 * 256;
 }

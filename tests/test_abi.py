@@ -304,3 +304,17 @@ def test_a_single_masked_pass_needs_no_workspace():
     assert lib.qsdpa_decode_range_bytes(ctypes.byref(a)) == 0
     a.bits = 3
     assert lib.qsdpa_decode_range_bytes(ctypes.byref(a)) == _lib.QSDPA_ERR_INVALID
+
+
+def test_key_ranges_only_where_workgroups_run_in_rounds():
+    """Workgroups that all run at once (at most one per CU, 256) take as long
+    as their longest row group: no ranges, nor with key splits."""
+    lib = _lib.load()
+    size = lambda **kw: lib.qsdpa_decode_range_bytes(ctypes.byref(_masked_prefill(**kw)))  # noqa: E731
+    assert size(B=2, Hq=32, Hkv=8, N=2048, L=512) == 0          # 16 groups x 16 heads
+    assert size(B=2, Hq=32, Hkv=8, N=2048, L=513) > 0           # 17 groups
+    assert size(B=1, Hq=16, Hkv=4, N=3000, L=64) == 0           # 8 workgroups: key splits
+    a = _masked_prefill(B=3, Hq=32, Hkv=8, N=2048, L=512)
+    assert lib.qsdpa_decode_range_bytes(ctypes.byref(a)) > 0
+    a.num_splits = 2
+    assert lib.qsdpa_decode_range_bytes(ctypes.byref(a)) == 0

@@ -443,12 +443,17 @@ def test_prefill_mask_shared_by_the_heads_gives_the_bits_of_one_each(device, D, 
     q, kq, vq = _inputs(B, Hq, Hkv, N, L, bits, gs, dtype, seed=N + 1, D=D)
     keep = _block_mask(B, L, N, seed=L + 1).to(device)
     print(f"prefill shared mask D={D} {dtype} N={N} L={L}", flush=True)
-    call = dict(scale=D ** -0.5, bits=bits, group_size=gs)
     args = (q, kq[0], vq[0], kq[1], vq[1], kq[2], vq[2])
-    shared = kernels.decode(*args, mask=keep, **call)
-    each = kernels.decode(*args, mask=keep.expand(B, Hq, L, N).contiguous(), **call)
-    torch.cuda.synchronize()
-    assert torch.equal(shared, each)
+    start = torch.tensor([77, 400, 0][:B], dtype=torch.int32, device=device)
+    add = torch.where(keep, 0.0, float("-inf")).to(dtype)
+    add[..., 100:140] += 2.0
+    for mask, kw in ((keep, {}), (keep, dict(causal=True, kv_start=start)), (add, {}), (add.float(), {}),
+                     (keep[:1], dict(kv_start=start)), (torch.zeros_like(keep), {}), (torch.ones_like(keep), {})):
+        call = dict(scale=D ** -0.5, bits=bits, group_size=gs, **kw)
+        shared = kernels.decode(*args, mask=mask, **call)
+        each = kernels.decode(*args, mask=mask.expand(B, Hq, L, N).contiguous(), **call)
+        torch.cuda.synchronize()
+        assert torch.equal(shared, each), (mask.dtype, kw)
 
 
 @pytest.mark.parametrize("bits,gs", [(4, 64), (8, 128)])
