@@ -357,7 +357,7 @@ struct Prefill {
 //
 // What it is worth (that chunk, 32 / 8 heads, 8-bit bf16, the call): 172 us
 // under the batch cache's mask against 202 over every tile.  What it costs: a
-// mask that leaves no tile out (all true, or holes everywhere) takes 219
+// mask that leaves no tile out (all true, or holes everywhere) takes 218
 // against 201.  Calls that cannot gain go without (prefill_range_bytes).  The
 // same look inside the prefill kernel, by each workgroup for itself, was 38 us
 // slower, a list there of the tiles with an attended key 27 us (and 42 us
@@ -514,23 +514,11 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
   const int T_all = (len + kTile - 1) / kTile;
   const int s_base = static_cast<int>(static_cast<int64_t>(split) * T_all / S);
   const int s_tiles = static_cast<int>(static_cast<int64_t>(split + 1) * T_all / S) - s_base;
-  // [j_base, j_base + T): those of them that the mask leaves (the cut itself
-  // does not follow the mask: split partials round, so moving it would move
-  // the output).
-  int j_base = s_base, T = s_tiles;
+  // The group's key ranges under the mask, in flight over the Q loads.
+  int2 range = int2{0, 0};
   if constexpr (MASK) {
-    if (p.ranges) {
-      const int2* rg = p.ranges + (static_cast<int64_t>(b) * groups_per_head + grp) * p.range_chunks;
-      const int2 x = lane < p.range_chunks ? rg[lane] : int2{0, 0};
-      const uint64_t m = __builtin_amdgcn_ballot_w64(x.y > 0);
-      int lo = 0, hi = 0;
-      if (m) {
-        lo = __builtin_amdgcn_readlane(x.x, static_cast<int>(__builtin_ctzll(m)));
-        hi = __builtin_amdgcn_readlane(x.y, 63 - static_cast<int>(__builtin_clzll(m)));
-      }
-      j_base = max(s_base, max(lo - s0, 0) / kTile);
-      T = max(min(s_base + s_tiles, (max(hi - s0, 0) + kTile - 1) / kTile) - j_base, 0);
-    }
+    if (p.ranges && lane < p.range_chunks)
+      range = p.ranges[(static_cast<int64_t>(b) * groups_per_head + grp) * p.range_chunks + lane];
   }
 
   // The lane's row: v = v_first + 16 wave + r (clamped to the last real row).
@@ -593,6 +581,23 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
     src.kb_sn = static_cast<uint32_t>(p.kb_sn * 2);
     src.vb_sn = static_cast<uint32_t>(p.vb_sn * 2);
     P::lanes(src, tid);
+  }
+
+  // [j_base, j_base + T): the split's tiles that the mask leaves (the cut
+  // itself does not follow the mask: split partials round, so moving it would
+  // move the output).
+  int j_base = s_base, T = s_tiles;
+  if constexpr (MASK) {
+    if (p.ranges) {
+      const uint64_t m = __builtin_amdgcn_ballot_w64(range.y > 0);
+      int lo = 0, hi = 0;
+      if (m) {
+        lo = __builtin_amdgcn_readlane(range.x, static_cast<int>(__builtin_ctzll(m)));
+        hi = __builtin_amdgcn_readlane(range.y, 63 - static_cast<int>(__builtin_clzll(m)));
+      }
+      j_base = max(s_base, max(lo - s0, 0) / kTile);
+      T = max(min(s_base + s_tiles, (max(hi - s0, 0) + kTile - 1) / kTile) - j_base, 0);
+    }
   }
 
   f4 acc[PG::NB];
