@@ -5,7 +5,8 @@
 // ctypes structs, slicing) they took 13 us (update), 9 us (views) and 13 us
 // (attention) of host time, more than the kernels of every short step: one
 // sequence over 4096 keys 35.2 us a step against 18.7 here, a window of four
-// 36.7 against 19.6.
+// 36.7 against 19.6; a decode under a mask tensor (two sequences of 16 / 4
+// 128-wide heads over 2000 keys) 25.3 against 10.1.
 //
 // Every function takes only what it can check in full: plain strided tensors
 // on one GPU with the shapes, types and strides the wrapper would accept as
@@ -208,15 +209,41 @@ PyObject* grown(PyObject*, PyObject* const* a, Py_ssize_t n) {
   END_HANDLE_TH_ERRORS
 }
 
+// A mask of 1 to 4 dimensions that broadcasts to [B, H, L, N] with its keys
+// adjacent, as x's mask; false for any other.
+bool mask_view(const at::Tensor& m, int64_t B, int64_t H, int64_t L, int64_t N, qsdpa_decode_args& x) {
+  switch (m.scalar_type()) {
+    case at::kBool: x.mask_dtype = QSDPA_BOOL; break;
+    case at::kHalf: x.mask_dtype = QSDPA_F16; break;
+    case at::kBFloat16: x.mask_dtype = QSDPA_BF16; break;
+    case at::kFloat: x.mask_dtype = QSDPA_F32; break;
+    default: return false;
+  }
+  const int64_t d = m.dim(), to[4] = {B, H, L, N};
+  if (d < 1 || d > 4 || m.size(d - 1) != N || (N > 1 && m.stride(d - 1) != 1)) return false;
+  int64_t stride[3] = {0, 0, 0};  // of a broadcast dimension: 0
+  for (int64_t i = 4 - d; i < 3; ++i) {
+    const int64_t size = m.size(i - (4 - d));
+    if (size != 1 && size != to[i]) return false;
+    if (size > 1) stride[i] = m.stride(i - (4 - d));
+  }
+  x.mask = {m.data_ptr(), stride[0], stride[1], 1};
+  x.mask_stride_q = stride[2];
+  return true;
+}
+
+// The counters at a workspace's start (include/qsdpa.h).
+constexpr int64_t kCounterBytes = 64 << 10;
+
 // decode(q, packed_k, packed_v, k_scales, v_scales, k_biases, v_biases,
-// scale, bits, group_size, kv_start, num_splits, causal, workspace, stream):
-// the output of qsdpa_decode without a mask; the workspace bytes it needs
-// (positive) when `workspace` (uint8, or None) is smaller; its negative
-// code; or None.
+// scale, bits, group_size, kv_start, num_splits, causal, workspace, stream,
+// mask): the output of qsdpa_decode; the workspace bytes it has use for
+// (positive) when `workspace` (uint8, or None) is smaller: the split-K
+// scratch, then a masked prefill's key ranges; its negative code; or None.
 PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   HANDLE_TH_ERRORS
   int64_t bits, gs, splits, stream;
-  if (n != 15 || !PyFloat_Check(a[7]) || !as_int(a[8], bits) || !as_int(a[9], gs) || !as_int(a[11], splits) ||
+  if (n != 16 || !PyFloat_Check(a[7]) || !as_int(a[8], bits) || !as_int(a[9], gs) || !as_int(a[11], splits) ||
       !as_int(a[14], stream) || !PyBool_Check(a[12]) || (bits != 4 && bits != 8) || gs <= 0)
     Py_RETURN_NONE;
   const at::Tensor* t[7];
@@ -259,6 +286,10 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
       Py_RETURN_NONE;
     x.kv_start = ks->data_ptr<int32_t>();
   }
+  if (a[15] != Py_None) {
+    const at::Tensor* m = plain(a[15]);
+    if (!m || m->device() != q.device() || !mask_view(*m, B, Hq, L, N, x)) Py_RETURN_NONE;
+  }
   x.num_splits = splits;
   x.q_len = L;
   x.causal = a[12] == Py_True;
@@ -266,17 +297,23 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   int32_t planned = 1;
   const int64_t ws = qsdpa_decode_workspace_size(&x, &planned);
   if (ws < 0) return PyLong_FromLongLong(ws);
-  if (ws > 0) {
+  const int64_t rb = x.mask.ptr && L > 1 ? qsdpa_decode_range_bytes(&x) : 0;
+  if (rb < 0) return PyLong_FromLongLong(rb);
+  const int64_t at_ranges = std::max<int64_t>(ws, kCounterBytes), total = rb > 0 ? at_ranges + rb : ws;
+  void* ranges = nullptr;
+  if (total > 0) {
     // A captured call takes a workspace of its own (the wrapper's general path).
     if (capturing(stream_of(stream))) Py_RETURN_NONE;
     const at::Tensor* w = a[13] == Py_None ? nullptr : plain(a[13]);
-    if (!w || w->device() != q.device() || static_cast<int64_t>(w->nbytes()) < ws) return PyLong_FromLongLong(ws);
+    if (!w || w->device() != q.device() || static_cast<int64_t>(w->nbytes()) < total)
+      return PyLong_FromLongLong(total);
     x.workspace = w->data_ptr();
-    x.workspace_bytes = w->nbytes();
+    x.workspace_bytes = ws;
+    if (rb > 0) ranges = static_cast<uint8_t*>(w->data_ptr()) + at_ranges;
   }
   at::Tensor out = at::empty(q.sizes(), q.options().requires_grad(false));
   x.out = view(out);
-  const int rc = qsdpa_decode(&x, stream_of(stream));
+  const int rc = qsdpa_decode_ranges(&x, ranges, rb, stream_of(stream));
   return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }

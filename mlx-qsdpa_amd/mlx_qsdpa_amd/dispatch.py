@@ -141,7 +141,8 @@ def quantized_sdpa(
     """
     # Calls whose tensors need no conversion go straight to the native host
     # path, which checks them itself; what it does not take comes back here.
-    if (mask is None or (isinstance(mask, str) and mask == "causal")) \
+    masked = isinstance(mask, torch.Tensor)
+    if (mask is None or (masked and mask.is_cuda) or (isinstance(mask, str) and mask == "causal")) \
             and threshold is None and num_splits is None and q.dim() == 4 and q.shape[3] in kernels.HEAD_DIMS:
         several = q.shape[2] > 1
         if not several or q.shape[3] != 64 or (packed_k.dim() == 4 and _d64_in_kernel(
@@ -151,7 +152,8 @@ def quantized_sdpa(
                                         v_biases if both else None,
                                         scale=q.shape[3] ** -0.5 if scale is None else scale, bits=bits,
                                         group_size=group_size, kv_start=kv_start,
-                                        causal=several and mask is not None)
+                                        causal=several and mask is not None and not masked,
+                                        mask=mask if masked else None)
             if out is not None:
                 return out
     B, H_q, qL, D, H_kv, N = _validate(q, packed_k, packed_v, bits, group_size)

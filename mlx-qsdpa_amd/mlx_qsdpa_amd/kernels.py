@@ -542,27 +542,27 @@ def _capture_workspace(device, nbytes):
 _TICKET_BYTES = 65536
 
 
-def _native_decode(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start, num_splits, causal):
+def _native_decode(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start, num_splits, causal, mask):
     """qsdpa_decode through the native host path: the output, its negative
     code, or None where that does not take the tensors."""
     stream = _stream(q)
     ws = _workspace(q.device, stream, 0)
     fn = _host().decode
-    out = fn(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start, num_splits, causal, ws, stream)
+    out = fn(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start, num_splits, causal, ws, stream, mask)
     if type(out) is int and out > 0:
         ws = _workspace(q.device, stream, out)
-        out = fn(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start, num_splits, causal, ws, stream)
+        out = fn(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start, num_splits, causal, ws, stream, mask)
     return out
 
 
-def decode_repeat(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size, kv_start=None, causal=False):
-    """A decode without mask or explicit split count whose tensors need no
+def decode_repeat(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size, kv_start=None, causal=False, mask=None):
+    """A decode without explicit split count whose tensors need no
     conversion, through the native host path; None for any other call, and
     for shapes that no kernel takes (the caller then takes the full path,
     which converts, falls back or raises)."""
     if not q.is_cuda:
         return None
-    out = _native_decode(q, pk, pv, ks, vs, kb, vb, float(scale), bits, group_size, kv_start, 0, causal)
+    out = _native_decode(q, pk, pv, ks, vs, kb, vb, float(scale), bits, group_size, kv_start, 0, causal, mask)
     return out if isinstance(out, torch.Tensor) else None
 
 
@@ -586,13 +586,13 @@ def decode(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size, mask=None, kv_
     key N - 1 of the caches before the attention (see DecodePlan).
     """
     _require_device(q, pk, pv, ks, vs, kb, vb, mask, kv_start, *(append or ()))
-    if mask is None and out is None and workspace is None and append is None and prof_events is None:
+    if out is None and workspace is None and append is None and prof_events is None:
         q = _inner_contig(q)
         if kv_start is not None and (kv_start.dtype != torch.int32 or kv_start.device != q.device
                                      or not kv_start.is_contiguous()):
             kv_start = kv_start.to(device=q.device, dtype=torch.int32).contiguous()
         res = _native_decode(q, pk, pv, ks, vs, kb, vb, float(scale), bits, group_size, kv_start, int(num_splits),
-                             bool(causal))
+                             bool(causal), mask)
         if res is not None:
             return res if isinstance(res, torch.Tensor) else _lib.check(res)
     q = _inner_contig(q)

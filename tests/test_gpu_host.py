@@ -33,6 +33,10 @@ def _both(monkeypatch, a):
     return got, want, isinstance(took[0], torch.Tensor) if took else False
 
 
+def _keep(*shape):
+    return torch.rand(shape, generator=torch.Generator(device="cuda").manual_seed(7), device="cuda") < 0.8
+
+
 def _off_by_one(t):
     wide = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
     wide[1:] = t.reshape(-1)
@@ -51,6 +55,18 @@ FORMS = {
     "q_2_bytes_off": ({}, lambda a: dict(a, q=_off_by_one(a["q"])), True),
     "codes_in_odd_rows": ({}, lambda a: dict(a, packed_k=torch.nn.functional.pad(
         a["packed_k"].view(torch.int32), (1, 0)).view(torch.uint32)[..., 1:]), False),
+    "bool": ({}, lambda a: dict(a, mask=_keep(2, 1, 1, 2000)), True),
+    "bool_rows": ({"L": 5}, lambda a: dict(a, mask=_keep(2, 8, 5, 2000)), True),
+    "bool_2d": ({"L": 5}, lambda a: dict(a, mask=_keep(5, 2000)), True),
+    "bool_1d_start": ({}, lambda a: dict(a, mask=_keep(2000), kv_start=torch.tensor([3, 700], dtype=torch.int32,
+                                                                                   device="cuda")), True),
+    "bool_view": ({}, lambda a: dict(a, mask=_keep(2, 1, 1, 2001)[..., 1:]), True),
+    "additive_f16": ({}, lambda a: dict(a, mask=_keep(1, 8, 1, 2000).half()), True),
+    "additive_bf16": ({"D": 256}, lambda a: dict(a, mask=_keep(2, 1, 1, 2000).bfloat16()), True),
+    "additive_f32": ({"D": 64}, lambda a: dict(a, mask=_keep(2, 1, 1, 2000).float()), True),
+    "mask_of_strided_keys": ({}, lambda a: dict(a, mask=_keep(2, 1, 1, 4000)[..., ::2]), False),
+    "host_mask": ({}, lambda a: dict(a, mask=_keep(2, 1, 1, 2000).cpu()), True),
+    "masked_prefill": ({"L": 700, "B": 12, "Hkv": 4}, lambda a: dict(a, mask=_keep(12, 1, 700, 2000)), True),
     "d256": ({"D": 256, "bits": 8, "dtype": torch.bfloat16}, lambda a: a, True),
 }
 
@@ -70,11 +86,15 @@ def test_native_decode_equals_the_general_path(device, monkeypatch, form):
     (lambda a: dict(a, k_scales=a["k_scales"].float()), ValueError),
     (lambda a: dict(a, kv_start=torch.zeros(3, dtype=torch.int32, device="cuda")), ValueError),
     (lambda a: dict(a, bits=3), ValueError),
+    (lambda a: dict(a, mask=_keep(2, 1, 1, 1999)), ValueError),
+    (lambda a: dict(a, mask=_keep(3, 1, 1, 2000)), RuntimeError),
+    (lambda a: dict(a, mask=_keep(2, 1, 2, 2000)), ValueError),
+    (lambda a: dict(a, mask=_keep(2, 1, 1, 2000).to(torch.int8)), ValueError),
     (lambda a: dict(a, q=a["q"].cpu()), RuntimeError),
     (lambda a: dict(a, packed_k=a["packed_k"][:, :, :0], packed_v=a["packed_v"][:, :, :0],
                     k_scales=a["k_scales"][:, :, :0], v_scales=a["v_scales"][:, :, :0],
                     k_biases=None, v_biases=None), RuntimeError),
-], ids=["shape", "codes", "scales", "start", "bits", "host", "empty"])
+], ids=["shape", "codes", "scales", "start", "bits", "mask_keys", "mask_batch", "mask_rows", "mask_type", "host", "empty"])
 def test_refusals(device, change, error):
     with pytest.raises(error):
         mq.quantized_sdpa(**change(_call()))
@@ -123,6 +143,26 @@ def test_captured_decode_replays(device):
         torch.cuda.synchronize()
         assert torch.equal(out, want)
         kernels._ARGS.d = {}  # the shared workspaces go; the graph's stays
+
+
+def test_captured_masked_prefill_replays(device):
+    """A captured masked prefill of several rounds keeps its key ranges in the
+    graph's own workspace."""
+    a = _call(B=12, Hkv=4, L=300, N=900)
+    a["mask"] = torch.ones(12, 1, 300, 900, dtype=torch.bool, device="cuda").tril(600)
+    want = mq.quantized_sdpa(**a)
+    other = dict(a, mask=_keep(12, 1, 300, 900))
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = mq.quantized_sdpa(**a)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        mq.quantized_sdpa(**other)
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        kernels._ARGS.d = {}
 
 
 def test_threads_on_one_stream(device):
