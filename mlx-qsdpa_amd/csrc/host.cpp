@@ -74,6 +74,17 @@ int dtype_of(const at::Tensor& t) {
 
 void* stream_of(int64_t x) { return reinterpret_cast<void*>(static_cast<intptr_t>(x)); }
 
+// The interpreter's lock is released over a launch, which may wait for room in
+// the stream's queue (as ctypes releases it on the general path).
+template <typename F>
+auto unlocked(F&& launch) {
+  struct Lock {
+    PyThreadState* state = PyEval_SaveThread();
+    ~Lock() { PyEval_RestoreThread(state); }
+  } lock;
+  return launch();
+}
+
 bool capturing(void* stream) {
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) != hipSuccess || st != hipStreamCaptureStatusNone;
@@ -114,7 +125,7 @@ PyObject* quantize_kv(PyObject*, PyObject* const* a, Py_ssize_t n) {
       !quantize_job(a[0], a[2], t0, bits, gs, j[0]) || !quantize_job(a[1], a[3], t0, bits, gs, j[1]) ||
       j[0].dtype != j[1].dtype || THPVariable_Unpack(a[0]).device() != THPVariable_Unpack(a[1]).device())
     Py_RETURN_NONE;
-  return PyLong_FromLong(qsdpa_quantize_batch(j, 2, stream_of(stream)));
+  return PyLong_FromLong(unlocked([&] { return qsdpa_quantize_batch(j, 2, stream_of(stream)); }));
   END_HANDLE_TH_ERRORS
 }
 
@@ -204,7 +215,7 @@ PyObject* grown(PyObject*, PyObject* const* a, Py_ssize_t n) {
     if (!o) return nullptr;
     PyTuple_SET_ITEM(out.get(), i, o);
   }
-  const int rc = qsdpa_move_rows(moves, count, stream_of(stream));
+  const int rc = unlocked([&] { return qsdpa_move_rows(moves, count, stream_of(stream)); });
   return rc ? PyLong_FromLong(rc) : out.release();
   END_HANDLE_TH_ERRORS
 }
@@ -313,7 +324,7 @@ PyObject* decode(PyObject*, PyObject* const* a, Py_ssize_t n) {
   }
   at::Tensor out = at::empty(q.sizes(), q.options().requires_grad(false));
   x.out = view(out);
-  const int rc = qsdpa_decode_ranges(&x, ranges, rb, stream_of(stream));
+  const int rc = unlocked([&] { return qsdpa_decode_ranges(&x, ranges, rb, stream_of(stream)); });
   return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -361,7 +372,7 @@ PyObject* causal_mask(PyObject*, PyObject* const* a, Py_ssize_t n) {
   x.start = start.data();
   x.pad = pad.empty() ? nullptr : pad.data();
   x.out = static_cast<uint8_t*>(out.data_ptr());
-  const int rc = qsdpa_causal_mask(&x, stream_of(stream));
+  const int rc = unlocked([&] { return qsdpa_causal_mask(&x, stream_of(stream)); });
   return rc ? PyLong_FromLong(rc) : THPVariable_Wrap(std::move(out));
   END_HANDLE_TH_ERRORS
 }
@@ -410,7 +421,7 @@ PyObject* rotate(PyObject*, PyObject* const* a, Py_ssize_t n) {
   x.start = start.data();
   x.q = view(*q); x.k = view(*k);
   x.q_out = view(out[0]); x.k_out = view(out[1]);
-  const int rc = qsdpa_rotate(&x, stream_of(stream));
+  const int rc = unlocked([&] { return qsdpa_rotate(&x, stream_of(stream)); });
   if (rc) return PyLong_FromLong(rc);
   THPObjectPtr pair(PyTuple_New(2));
   if (!pair) return nullptr;

@@ -1,11 +1,15 @@
 """The native host path (csrc/host.cpp) against the wrappers' general path."""
 
+import shutil
+import subprocess
+import sys
 import threading
 
 import pytest
 import torch
 
 import mlx_qsdpa_amd as mq
+from conftest import ROOT
 from mlx_qsdpa_amd import kernels
 
 pytestmark = pytest.mark.gpu
@@ -181,3 +185,51 @@ def test_threads_on_one_stream(device):
     [t.start() for t in ts]
     [t.join() for t in ts]
     assert not bad
+
+
+# The library's launches replaced: each returns an error while its thread
+# holds the interpreter's lock.
+_STUB = """
+#include "qsdpa.h"
+extern "C" {
+int PyGILState_Check(void);
+static int held() { return PyGILState_Check() ? QSDPA_ERR_LAUNCH : QSDPA_OK; }
+int qsdpa_abi_version(void) { return QSDPA_ABI_VERSION; }
+int64_t qsdpa_decode_workspace_size(const qsdpa_decode_args*, int32_t*) { return 0; }
+int64_t qsdpa_decode_range_bytes(const qsdpa_decode_args*) { return 0; }
+int qsdpa_decode(const qsdpa_decode_args*, void*) { return held(); }
+int qsdpa_decode_ranges(const qsdpa_decode_args*, void*, int64_t, void*) { return held(); }
+int qsdpa_quantize_batch(const qsdpa_quantize_args*, int32_t, void*) { return held(); }
+int qsdpa_move_rows(const qsdpa_row_move*, int32_t, void*) { return held(); }
+int qsdpa_causal_mask(const qsdpa_causal_mask_args*, void*) { return held(); }
+int qsdpa_rotate(const qsdpa_rotate_args*, void*) { return held(); }
+}
+"""
+
+_CHILD = """
+import sys, torch
+torch.zeros(1, device="cuda")
+sys.path.insert(0, sys.argv[1])
+import _host
+x = torch.zeros(1, 2, 4, 64, dtype=torch.float16, device="cuda")
+b = tuple(torch.zeros(1, 2, 4, w, dtype=t, device="cuda") for w, t in ((8, torch.uint32), (2, x.dtype), (2, x.dtype)))
+out = {"quantize_kv": _host.quantize_kv(x, x, b, b, 0, 4, 32, 0),
+       "grown": _host.grown(x, x, None, 0, 8, 4, 32, 0),
+       "decode": _host.decode(x, b[0], b[0], b[1], b[1], b[2], b[2], 1.0, 4, 32, None, 0, False, None, 0, None),
+       "rotate": _host.rotate(x, x, 3, 1e4, 0),
+       "causal_mask": _host.causal_mask(4, 3, None, None, 0, 0)}
+for name, got in out.items():
+    assert got is not None and (got == 0 if name == "quantize_kv" else type(got) is not int), name
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_launches_release_the_interpreter(device, tmp_path):
+    """Every native call gives the interpreter's lock back around its launch
+    (a launch waits when the stream's queue is full)."""
+    lib, host = tmp_path / "libqsdpa_hip.so", ROOT / "mlx-qsdpa_amd" / "mlx_qsdpa_amd" / "_host.so"
+    (tmp_path / "stub.cpp").write_text(_STUB)
+    subprocess.run(["g++", "-shared", "-fPIC", f"-I{ROOT / 'include'}", str(tmp_path / "stub.cpp"), "-o", str(lib)],
+                   check=True)
+    shutil.copy(host, tmp_path / "_host.so")
+    subprocess.run([sys.executable, "-c", _CHILD, str(tmp_path)], check=True, timeout=100)
