@@ -222,7 +222,7 @@ def requant_window(old: tuple, new: tuple, dst: tuple, n_old: int, keep: int, ro
 
 def columns(buffers: tuple, n: int) -> tuple:
     """The first n columns (dim 2) of each of a cache's (B, H, N, W) tensors."""
-    out = _host().columns(buffers, n)
+    out = _host().columns(buffers, n) if buffers[0].is_cuda else None
     return tuple(t[:, :, :n, :] for t in buffers) if out is None else out
 
 

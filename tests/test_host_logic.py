@@ -438,3 +438,14 @@ def test_growth_rejects_other_shapes(cpu_kernels, rng):
     c.update_and_fetch(*_kv(rng, 2, 3, 256, 64))
     with pytest.raises(RuntimeError):
         c.update_and_fetch(*_kv(rng, 3, 2, 256, 64))
+
+
+def test_caches_on_the_cpu_need_no_library(cpu_kernels, rng, monkeypatch):
+    """Slices of CPU buffers (state, trim, what an update returns) are torch's
+    alone: no built library."""
+    monkeypatch.setattr(pc.kernels, "_host", None)
+    for c in (pc.QuantizedSDPACache(bits=4, group_size=32), pc.BatchQuantizedSDPACache([0, 0], bits=4, group_size=32)):
+        k, v = _kv(rng, 2, 3, 300, 64)
+        got, _ = c.update_and_fetch(k, v)
+        c.trim(5)
+        assert got[0].shape[2] == 300 and all(t.shape[2] == 295 for t in c.state[0])
