@@ -453,4 +453,9 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, methods, null
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__host() { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__host() {
+  if (qsdpa_abi_version() != QSDPA_ABI_VERSION)
+    return PyErr_Format(PyExc_ImportError, "_host.so was built for ABI version %d of libqsdpa_hip.so, found %d",
+                        QSDPA_ABI_VERSION, qsdpa_abi_version());
+  return PyModule_Create(&module);
+}

@@ -80,7 +80,11 @@ def _host():
     global _HOST
     if _HOST is None:
         _lib.load()  # says what to build when it is missing
-        from . import _host as mod
+        try:
+            from . import _host as mod
+        except ImportError as e:
+            raise ImportError(f"the native host path does not load ({e}): build it, with the library, by "
+                              "`python mlx-qsdpa_amd/build_lib.py`") from e
         _HOST = mod
     return _HOST
 

@@ -11,6 +11,7 @@ import ctypes
 import re
 import shutil
 import subprocess
+import sys
 
 import pytest
 import torch
@@ -318,3 +319,28 @@ def test_key_ranges_only_where_workgroups_run_in_rounds():
     assert lib.qsdpa_decode_range_bytes(ctypes.byref(a)) > 0
     a.num_splits = 2
     assert lib.qsdpa_decode_range_bytes(ctypes.byref(a)) == 0
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="g++ not available")
+def test_native_host_path_refuses_another_abi(tmp_path):
+    """_host.so reads the argument structs of the version it was built for:
+    beside a library of another one it does not load."""
+    names = [n for n in _declared_functions() if n != "qsdpa_abi_version"]
+    src = 'extern "C" {\n' + "".join(f"int {n}(void) {{ return 0; }}\n" for n in names)
+    src += f"int qsdpa_abi_version(void) {{ return {_lib.ABI_VERSION - 1}; }}\n}}\n"
+    (tmp_path / "stub.cpp").write_text(src)
+    subprocess.run(["g++", "-shared", "-fPIC", str(tmp_path / "stub.cpp"), "-o", str(tmp_path / "libqsdpa_hip.so")],
+                   check=True)
+    shutil.copy(_lib.LIB_PATH.parent / "_host.so", tmp_path)
+    code = f"import sys, torch; sys.path.insert(0, {str(tmp_path)!r}); import _host"
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100)
+    assert r.returncode != 0 and "ImportError" in r.stderr and f"found {_lib.ABI_VERSION - 1}" in r.stderr
+
+
+def test_a_missing_host_path_names_what_to_build(monkeypatch):
+    from mlx_qsdpa_amd import kernels
+    monkeypatch.setattr(kernels, "_HOST", None)
+    monkeypatch.setitem(sys.modules, "mlx_qsdpa_amd._host", None)
+    monkeypatch.delattr("mlx_qsdpa_amd._host", raising=False)
+    with pytest.raises(ImportError, match="build_lib.py"):
+        kernels._host()
