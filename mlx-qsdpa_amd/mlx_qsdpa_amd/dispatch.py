@@ -148,7 +148,7 @@ def quantized_sdpa(
         if not several or q.shape[3] != 64 or (packed_k.dim() == 4 and _d64_in_kernel(
                 mask, kv_start, q.shape[0], q.shape[1], q.shape[2], packed_k.shape[2])):
             both = k_biases is not None and v_biases is not None
-            out = kernels.decode_repeat(q, packed_k, packed_v, k_scales, v_scales, k_biases if both else None,
+            out = kernels.decode_native(q, packed_k, packed_v, k_scales, v_scales, k_biases if both else None,
                                         v_biases if both else None,
                                         scale=q.shape[3] ** -0.5 if scale is None else scale, bits=bits,
                                         group_size=group_size, kv_start=kv_start,

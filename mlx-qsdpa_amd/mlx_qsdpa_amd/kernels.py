@@ -559,15 +559,20 @@ def _native_decode(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start,
     return out
 
 
-def decode_repeat(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size, kv_start=None, causal=False, mask=None):
+def decode_native(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size, kv_start=None, causal=False, mask=None):
     """A decode without explicit split count whose tensors need no
     conversion, through the native host path; None for any other call, and
-    for shapes that no kernel takes (the caller then takes the full path,
-    which converts, falls back or raises)."""
+    for arguments that no kernel takes (the caller then takes the full path,
+    which converts, falls back or raises).  Any other failure, a launch's
+    among them, raises: the launch is not tried again."""
     if not q.is_cuda:
         return None
     out = _native_decode(q, pk, pv, ks, vs, kb, vb, float(scale), bits, group_size, kv_start, 0, causal, mask)
-    return out if isinstance(out, torch.Tensor) else None
+    if type(out) is int:
+        if out not in (_lib.QSDPA_ERR_INVALID, _lib.QSDPA_ERR_UNSUPPORTED):
+            _lib.check(out)
+        return None
+    return out
 
 
 def decode(q, pk, pv, ks, vs, kb, vb, *, scale, bits, group_size, mask=None, kv_start=None,

@@ -388,7 +388,7 @@ def test_uncompiled_head_dims(device, monkeypatch, D, bits, gs, dt):
         raise AssertionError("the fused kernel ran")
 
     monkeypatch.setattr(kernels, "decode", no_fused)
-    monkeypatch.setattr(kernels, "decode_repeat", no_fused)
+    monkeypatch.setattr(kernels, "decode_native", no_fused)
     for L in (1, 3):
         q = affine.random_T(rng, (B, Hq, L, D), dt)
         for mask in (None, "bool", "additive", "causal"):

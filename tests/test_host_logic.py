@@ -449,3 +449,19 @@ def test_caches_on_the_cpu_need_no_library(cpu_kernels, rng, monkeypatch):
         got, _ = c.update_and_fetch(k, v)
         c.trim(5)
         assert got[0].shape[2] == 300 and all(t.shape[2] == 295 for t in c.state[0])
+
+
+def test_a_failed_native_launch_is_not_repeated(monkeypatch):
+    """The native host path's errors: arguments that no kernel takes go on to
+    the full path, a failed launch raises."""
+    from types import SimpleNamespace
+    from mlx_qsdpa_amd import _lib, kernels
+    q = SimpleNamespace(is_cuda=True)
+    call = lambda: kernels.decode_native(q, *[None] * 6, scale=1.0, bits=4, group_size=32)  # noqa: E731
+    for code in (_lib.QSDPA_ERR_INVALID, _lib.QSDPA_ERR_UNSUPPORTED):
+        monkeypatch.setattr(kernels, "_native_decode", lambda *a: code)
+        assert call() is None
+    for code in (_lib.QSDPA_ERR_LAUNCH, _lib.QSDPA_ERR_WORKSPACE):
+        monkeypatch.setattr(kernels, "_native_decode", lambda *a: code)
+        with pytest.raises(_lib.QsdpaError):
+            call()
