@@ -95,10 +95,11 @@ def _heads_as_rows(t):
     return t.as_strided((1, B * H, N, W), (0, t.stride(1), t.stride(2), t.stride(3)))
 
 
-def _grow(cache, keys, values, prev):
-    """Room for the new tokens after the first `prev` (cache.py:199-231):
-    ceil(S / step) * step more columns than the buffers hold, trimmed to prev
-    first unless that is a multiple of the step.  One launch copies the held
+def _grown(cache, keys, values, prev):
+    """Buffers (of the keys, of the values) with room for the new tokens after
+    the first `prev` (cache.py:199-231): ceil(S / step) * step more columns
+    than the cache's hold, trimmed to prev first unless that is a multiple of
+    the step.  The cache's own stay as they are.  One launch copies the held
     columns and zeroes those past the new tokens, which the caller writes next
     (zero-filling new buffers whole and concatenating took a launch or two for
     each of the six tensors and a pass over the columns about to be written:
@@ -114,8 +115,7 @@ def _grow(cache, keys, values, prev):
     cols = base + new_alloc
     new = kernels.grown(keys, values, old, prev, cols, cache.bits, cache.group_size)
     if new is not None:
-        cache._keys, cache._values = new[:3], new[3:]
-        return
+        return new[:3], new[3:]
     new, moves = [], []
     for x in (keys, values):
         W = x.shape[3]
@@ -133,7 +133,18 @@ def _grow(cache, keys, values, prev):
             else:
                 moves += [kernels.RowMove(d, b, 0, prev, old[i], b, 0, 0, prev) for b in range(B)]
     kernels.move_rows(moves)
-    cache._keys, cache._values = tuple(new[:3]), tuple(new[3:])
+    return tuple(new[:3]), tuple(new[3:])
+
+
+def _append(cache, keys, values, prev):
+    """Quantize the new tokens into columns [prev, prev + S) of the cache's
+    buffers, or of grown ones, which it holds only once that is done: an
+    update that raises leaves the cache as it was."""
+    held = cache._keys, cache._values
+    if held[0] is None or prev + keys.shape[2] > held[0][0].shape[2]:
+        held = _grown(cache, keys, values, prev)
+    kernels.quantize_kv_into(keys, values, *held, prev, cache.bits, cache.group_size)
+    cache._keys, cache._values = held
 
 
 def _ring_runs(keep, ptr, n):
@@ -338,13 +349,8 @@ class QuantizedSDPACache:
 
     def update_and_fetch(self, keys, values):
         """Quantize keys/values (B, H_kv, S, D) and append them (cache.py:163-197)."""
-        S = keys.shape[2]
-        prev = self.offset
-        if self._keys is None or prev + S > self._keys[0].shape[2]:
-            _grow(self, keys, values, prev)
-        self.offset += S
-        kernels.quantize_kv_into(keys, values, self._keys, self._values, prev, self.bits,
-                                 self.group_size)
+        _append(self, keys, values, self.offset)
+        self.offset += keys.shape[2]
         return _sl(self._keys, 0, self.offset), _sl(self._values, 0, self.offset)
 
 
@@ -401,13 +407,9 @@ class BatchQuantizedSDPACache:
     def update_and_fetch(self, keys, values):
         """cache.py:279-322: all sequences append at the shared column _idx."""
         S = keys.shape[2]
-        prev = self._idx
-        if self._keys is None or prev + S > self._keys[0].shape[2]:
-            _grow(self, keys, values, prev)
+        _append(self, keys, values, self._idx)
         self.offset = self.offset + S
         self._idx += S
-        kernels.quantize_kv_into(keys, values, self._keys, self._values, prev, self.bits,
-                                 self.group_size)
         return _sl(self._keys, 0, self._idx), _sl(self._values, 0, self._idx)
 
     def prepare(self, *, left_padding=None, lengths=None, right_padding=None):

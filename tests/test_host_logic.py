@@ -465,3 +465,27 @@ def test_a_failed_native_launch_is_not_repeated(monkeypatch):
         monkeypatch.setattr(kernels, "_native_decode", lambda *a: code)
         with pytest.raises(_lib.QsdpaError):
             call()
+
+
+@pytest.mark.parametrize("held", [0, 256, 300])
+@pytest.mark.parametrize("batch", [False, True])
+def test_a_rejected_update_leaves_the_cache_as_it_was(cpu_kernels, rng, monkeypatch, held, batch):
+    """An update whose quantization raises (here: always) counts no tokens and
+    keeps the buffers, whether it grows them or not."""
+    c = pc.BatchQuantizedSDPACache([0, 0], bits=4, group_size=32) if batch else pc.QuantizedSDPACache(4, 32)
+    if held:
+        c.update_and_fetch(*_kv(rng, 2, 3, held, 64))
+    keys, values = c._keys, c._values
+    before = (int(c._idx), c.offset.tolist()) if batch else c.offset
+
+    def refuse(*a):
+        raise ValueError("refused")
+
+    with monkeypatch.context() as m:
+        m.setattr(pc.kernels, "quantize_kv_into", refuse)
+        with pytest.raises(ValueError):
+            c.update_and_fetch(*_kv(rng, 2, 3, 5, 64))
+    assert c._keys is keys and c._values is values
+    assert before == ((int(c._idx), c.offset.tolist()) if batch else c.offset)
+    c.update_and_fetch(*_kv(rng, 2, 3, 5, 64))
+    assert c._keys[0].shape[2] >= held + 5
