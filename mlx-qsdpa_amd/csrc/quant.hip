@@ -94,11 +94,14 @@ __global__ __launch_bounds__(256) void quantize_kernel(QuantJobs jobs) {
                                    p.db + off3(b, h, t, p.z_sb, p.z_sh, p.z_sn) + g);
 }
 
-// Jobs with at least this many groups take GS / 32 lanes per group.  Whole
-// passes with GS / 8 against GS / 32 lanes: a 3000-token prompt (48000 groups
-// of 64, 4-bit) 132.1 against 130.7 us, 500 tokens onto 8 sequences (64000,
-// 8-bit) 175.4 against 173.2, a 1500-token prompt (12000) 42.55 against 43.1.
-constexpr int64_t kWideJobGroups = 1 << 15;
+// Jobs with at least this many values take GS / 32 lanes per group: the forms
+// cross where the wide one's lanes (32 values each) still fill the GPU, at
+// the same number of values for every group size, type and width.  K and V of
+// 2^20 / 2^21 / 2^22 values each, GS / 8 lanes against GS / 32: float16 4-bit
+// 4.11 / 6.05 / 9.78 us against 3.97 / 5.24 / 7.32 (groups of 64; of 32 and
+// 128 within 4%), bfloat16 8-bit 4.20 / 6.49 / 10.18 against 4.68 / 5.95 /
+// 8.23; 3 * 2^19 values 0.97 to 1.06 times as fast.
+constexpr int64_t kWideJobValues = 1 << 21;
 
 template <typename Tag, int BITS, int GS, int L>
 void launch_quantize_l(const QuantJobs& j, bool vec, int64_t groups, int count, hipStream_t stream) {
@@ -115,7 +118,7 @@ void launch_quantize_l(const QuantJobs& j, bool vec, int64_t groups, int count, 
 
 template <typename Tag, int BITS, int GS>
 void launch_quantize_gs(const QuantJobs& j, bool vec, int64_t groups, int count, hipStream_t stream) {
-  if (groups >= kWideJobGroups) launch_quantize_l<Tag, BITS, GS, GS / 32>(j, vec, groups, count, stream);
+  if (groups * GS >= kWideJobValues) launch_quantize_l<Tag, BITS, GS, GS / 32>(j, vec, groups, count, stream);
   else launch_quantize_l<Tag, BITS, GS, GS / 8>(j, vec, groups, count, stream);
 }
 

@@ -50,10 +50,30 @@ def test_quantize_kernel_matches_oracle(device, dtype, bits, gs, D):
     assert _bits_equal(to_np(got[2]), want[2], dtype)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("bits,gs", [(4, 32), (8, 64), (4, 128)])
+def test_quantize_on_both_sides_of_the_line(device, dtype, bits, gs):
+    """A job of 2^21 values (32 to a lane), of one row less (8 to a lane), and
+    the same rows in small jobs: the same bits; rows off the 16-byte grid too."""
+    rows, D = (1 << 21) // 128, 128
+    x = torch.randn(rows, D + 1, generator=torch.Generator(device="cuda").manual_seed(gs), device=device).to(dtype)
+    for w in (x[:, :D].contiguous(), x[:, 1:]):
+        w4 = w[None, None]
+        outs = []
+        for cuts in ((0, rows), (0, rows - 1, rows), (0, 1000, rows // 3, rows // 2, rows)):
+            dst = (torch.zeros(1, 1, rows, D * bits // 32, dtype=torch.uint32, device=device),
+                   *(torch.zeros(1, 1, rows, D // gs, dtype=dtype, device=device) for _ in range(2)))
+            for lo, hi in zip(cuts, cuts[1:]):
+                kernels.quantize_into(w4[:, :, lo:hi], dst, lo, bits, gs)
+            outs.append(dst)
+        torch.cuda.synchronize()
+        for o in outs[1:]:
+            assert all(torch.equal(a.view(torch.int16), b.view(torch.int16)) for a, b in zip(outs[0], o))
+
+
 @pytest.mark.parametrize("dtype,bits,gs", [("f16", 4, 32), ("bf16", 8, 64)])
 def test_quantize_bulk_matches_oracle(device, dtype, bits, gs):
-    """A prompt-sized job (>= 2^18 groups) takes the one-lane-per-group
-    kernel; bit-exact like the per-token appends."""
+    """A prompt-sized job takes GS / 32 lanes per group; bit-exact like the per-token appends."""
     rng = np.random.default_rng(bits * 7 + gs)
     D = 128
     S = (1 << 18) * gs // D // 8  # 8 heads x S rows x D / gs groups = 2^18
