@@ -253,9 +253,9 @@ __device__ __forceinline__ void decode_segment(const MfmaParams& p, float* s_acc
 
   const int64_t mrow = static_cast<int64_t>(b) * p.m_sb + static_cast<int64_t>(hq_lane) * p.m_sh +
                        static_cast<int64_t>(iq_lane) * p.m_sq;  // the lane's mask row
-  f4 acc[G::NB];
+  f4 acc[K::NA];
 #pragma unroll
-  for (int i = 0; i < G::NB; ++i) acc[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int i = 0; i < K::NA; ++i) acc[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
   float mrun = kNegBig;
   float lrun = 0.0f;
 
@@ -266,6 +266,11 @@ __device__ __forceinline__ void decode_segment(const MfmaParams& p, float* s_acc
     auto iv = [&](typename K::Regs& X) { K::load_v(X, rs, L, nrow); };
     K::template compute_tile<MASK>(R, p, qt, acc, mrun, lrun, s0 + row_of(j), s0, n_lane, quad, mrow, vm, ik, iv);
     j = nj;
+  }
+
+  if constexpr (K::kLo) {
+#pragma unroll
+    for (int i = 0; i < G::NB; ++i) acc[i] = join_terms(acc[i], acc[G::NB + i]);
   }
 
   // ---- per-head totals over the four quads ----

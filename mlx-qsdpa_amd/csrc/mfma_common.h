@@ -29,6 +29,25 @@ constexpr bool half_parts() {
   return Tag::kId == QSDPA_F16 && D != 64;
 }
 
+// D = 64 with float16 P.V operands: P (at most 2^kRescale) is scaled by
+// 2^kPShift, to the top of float16's range, and enters as its float16 value
+// and 2^11 times what that leaves, in accumulators of their own (join_terms).
+// A weight, as a share of the row's largest, is then off by at most 2^-23 of
+// itself or 2^-43 (16-bit results keep their bits down to weights of 2^-31):
+// with both terms in one accumulator, unscaled, by 2^-25, a percent and more
+// of the weights of 2^-21 beside an attention sink.
+constexpr float kPShift = 7.0f;
+constexpr float kLoScale = 2048.0f;
+
+// The sum of the two terms' accumulators.  An infinite first term (a V value
+// past float16's range) is the sum: the second's sign is any.
+__device__ __forceinline__ f4 join_terms(f4 hi, f4 lo) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    hi[i] = fabsf(hi[i]) == __builtin_huge_valf() ? hi[i] : fmaf(lo[i], 1.0f / kLoScale, hi[i]);
+  return hi;
+}
+
 struct MfmaParams {
   int B, Hq, Hkv, N, G, hb_count, num_splits;
   float qscale;  // softmax scale * log2(e)

@@ -33,9 +33,10 @@ struct Geo {
   // lanes 2i and 2i + 1 load one word and each takes its half.
   static constexpr bool HalfV = NB * BITS < 32;
   static constexpr int VW = HalfV ? 1 : NB * BITS / 32;  // V words per lane per token
-  // D = 64: P enters P.V as two 16-bit terms for float16 too, and split
-  // partials stay float32 (the kernel that these calls took before, and the
-  // dequantize + attention path of several positions, keep both in 32 bits).
+  // D = 64 holds P in float32, as the VALU kernel and the dequantize +
+  // attention path of several positions do: it enters P.V as two float16
+  // terms (kPShift) or three bfloat16 ones (24 bits), and split partials stay
+  // float32.
   static constexpr bool Wide = D == 64;
   static constexpr int RW = D * BITS / 32;      // words per row
   static constexpr int NG = D / GS;             // groups (scales) per row
@@ -177,6 +178,9 @@ struct Kernel {
   static constexpr int kAux = load_policy<D, BITS>();
   using G = Geo<D, BITS, GS>;
   using Regs = TileRegs<D, BITS, GS>;
+  // Accumulators: a second set for P's second term (kPShift).
+  static constexpr bool kLo = G::Wide && Tag::kId == QSDPA_F16;
+  static constexpr int NA = kLo ? 2 * G::NB : G::NB;
   // Every K / V element is dequantized as mx.dequantize rounds it, T(fma(
   // scale, code, bias)): float16 builds the code as an exact half (the
   // 1024 + code bit trick, minus 1024) and uses one v_pk_fma_f16 per pair.
@@ -284,7 +288,7 @@ struct Kernel {
   template <typename IV>
   static __device__ __forceinline__ void pv_f16(Regs& R, const uint32_t (&sv2)[4], const uint32_t (&bv2)[4],
                                                 const uint32_t (&pb)[4], const uint32_t (&pb_lo)[4], uint32_t vsel,
-                                                f4 (&acc)[G::NB], IV&& issue_v) {
+                                                f4 (&acc)[NA], IV&& issue_v) {
     if constexpr (G::HalfV) {
       // X: the lane's 4 nibbles of tokens (2i, 2i+1).
       uint32_t X[4];
@@ -297,7 +301,7 @@ struct Kernel {
 #pragma unroll
         for (int i = 0; i < 4; ++i) a[i] = f16x2_fma(nib_codes(X[i], X[i] >> 8, nb), sv2[i], bv2[i]);
         acc[nb] = mfma<Tag>(a, pb, acc[nb]);
-        acc[nb] = mfma<Tag>(a, pb_lo, acc[nb]);
+        acc[G::NB + nb] = mfma<Tag>(a, pb_lo, acc[G::NB + nb]);
       }
     } else if constexpr (BITS == 4) {
       // X: nibbles 0-3 of tokens (2i, 2i+1), Y: nibbles 4-7.
@@ -342,7 +346,7 @@ struct Kernel {
           a[i] = f16x2_fma(f16x2_sub1024(t), sv2[i], bv2[i]);
         }
         acc[nb] = mfma<Tag>(a, pb, acc[nb]);
-        if constexpr (G::Wide) acc[nb] = mfma<Tag>(a, pb_lo, acc[nb]);
+        if constexpr (kLo) acc[G::NB + nb] = mfma<Tag>(a, pb_lo, acc[G::NB + nb]);
       }
     }
   }
@@ -355,7 +359,7 @@ struct Kernel {
   // operands' pre-permuted form, so one register set suffices.
   template <bool MASK, typename IK, typename IV>
   static __device__ __forceinline__ void compute_tile(Regs& R, const MfmaParams& p, const uint32_t (&qt)[G::NM][4],
-                                                      f4 (&acc)[G::NB], float& mrun, float& lrun, int tb, int n0,
+                                                      f4 (&acc)[NA], float& mrun, float& lrun, int tb, int n0,
                                                       int n1, int quad, int64_t mrow, const VMetaLane& vm,
                                                       IK&& issue_k, IV&& issue_v) {
     // Mask values of the lane's 8 keys, loaded before the next tile's K
@@ -407,22 +411,26 @@ struct Kernel {
       mrun = mnew;
       lrun *= f;
 #pragma unroll
-      for (int i = 0; i < G::NB; ++i) acc[i] *= f;
+      for (int i = 0; i < NA; ++i) acc[i] *= f;
     }
+    const float nm = kLo ? kPShift - mrun : -mrun;
     float pr[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) pr[j] = fast_exp2(fmaf(sc[j], ea, -mrun));
+    for (int j = 0; j < 8; ++j) pr[j] = fast_exp2(fmaf(sc[j], ea, nm));
     lrun += ((pr[0] + pr[1]) + (pr[2] + pr[3])) + ((pr[4] + pr[5]) + (pr[6] + pr[7]));
 
     // ---- P^T operand: k slot 2i, 2i+1 = tokens tau(quad, 2i), tau(quad, 2i+1) ----
-    uint32_t pb[4], pb_lo[4];
+    uint32_t pb[4], pb_lo[4], pb_lo2[4];  // (pb_lo2: the third bfloat16 term)
 #pragma unroll
     for (int i = 0; i < 4; ++i) pb[i] = pack_T2<Tag>(pr[2 * i], pr[2 * i + 1]);
-    if constexpr (Tag::kId == QSDPA_BF16 || G::Wide) {
+    if constexpr (Tag::kId == QSDPA_BF16 || kLo) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        pb_lo[i] = pack_T2<Tag>(pr[2 * i] - unpack_T2_lo<Tag>(pb[i]),
-                                pr[2 * i + 1] - unpack_T2_hi<Tag>(pb[i]));
+      for (int i = 0; i < 4; ++i) {
+        const float x = pr[2 * i] - unpack_T2_lo<Tag>(pb[i]), y = pr[2 * i + 1] - unpack_T2_hi<Tag>(pb[i]);
+        pb_lo[i] = kLo ? pack_T2<Tag>(x * kLoScale, y * kLoScale) : pack_T2<Tag>(x, y);
+        if constexpr (G::Wide && !kLo)
+          pb_lo2[i] = pack_T2<Tag>(x - unpack_T2_lo<Tag>(pb_lo[i]), y - unpack_T2_hi<Tag>(pb_lo[i]));
+      }
     }
 
     // ---- out^T += V^T P^T: MFMA nb takes dim r*NB + nb of the lane's tokens ----
@@ -484,6 +492,7 @@ struct Kernel {
         }
         acc[nb] = mfma<Tag>(a, pb, acc[nb]);
         acc[nb] = mfma<Tag>(a, pb_lo, acc[nb]);
+        if constexpr (G::Wide) acc[nb] = mfma<Tag>(a, pb_lo2, acc[nb]);
       }
       issue_v(R);
     }

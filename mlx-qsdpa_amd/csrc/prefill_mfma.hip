@@ -97,7 +97,7 @@ constexpr float kPVSingle = 8.0f;
 // per tile, the same MFMA work too but for D = 64's second P term.
 //
 // D = 64 keeps what the dequantize + float32 attention path of these calls
-// held in 32 bits: P always enters P.V as two float16 terms (22 bits), split
+// held in 32 bits: P always enters P.V as two float16 terms (kPShift), split
 // partials are float32, a bfloat16 V is scaled to the top of float16's range
 // whatever its magnitude, and a row whose sum is NaN is zero.  Softmax bound:
 // twice the exponentials per MFMA of D = 128.
@@ -600,9 +600,12 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
     }
   }
 
-  f4 acc[PG::NB];
+  // D = 64: P scaled, and a second set of accumulators for its second term.
+  constexpr bool kLo = D == 64;
+  constexpr int NA = kLo ? 2 * PG::NB : PG::NB;
+  f4 acc[NA];
 #pragma unroll
-  for (int i = 0; i < PG::NB; ++i) acc[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int i = 0; i < NA; ++i) acc[i] = f4{0.0f, 0.0f, 0.0f, 0.0f};
   float mrun = kNegBig, lrun = 0.0f;
   float vsc = 1.0f, osc = 1.0f;  // V scale 2^-k in LDS, output scale 2^k (bfloat16)
 
@@ -695,9 +698,9 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
       mrun = mnew;
       lrun *= f;
 #pragma unroll
-      for (int i = 0; i < PG::NB; ++i) acc[i] *= f;
+      for (int i = 0; i < NA; ++i) acc[i] *= f;
     }
-    const float nm = -mrun;
+    const float nm = kLo ? kPShift - mrun : -mrun;
     float pr[NE];
 #pragma unroll
     for (int e = 0; e < NE; ++e) pr[e] = fast_exp2(fmaf(sc[e], ea, nm));
@@ -716,8 +719,10 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
       for (int i = 0; i < 4; ++i) {
         const int e = 4 * (2 * u + (i >> 1)) + 2 * (i & 1);
         pb[u][i] = pack_T2<F16>(pr[e], pr[e + 1]);
-        if constexpr (kTwo)
-          pl[u][i] = pack_T2<F16>(pr[e] - unpack_T2_lo<F16>(pb[u][i]), pr[e + 1] - unpack_T2_hi<F16>(pb[u][i]));
+        if constexpr (kTwo) {
+          const float x = pr[e] - unpack_T2_lo<F16>(pb[u][i]), y = pr[e + 1] - unpack_T2_hi<F16>(pb[u][i]);
+          pl[u][i] = kLo ? pack_T2<F16>(x * kLoScale, y * kLoScale) : pack_T2<F16>(x, y);
+        }
       }
     // ---- out^T += V^T P^T (two terms: the hi terms of all dim blocks, then the lo terms) ----
     const uint8_t* vt = cur + PG::KBytes;
@@ -732,7 +737,10 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
       }
       if constexpr (kTwo) {
 #pragma unroll
-        for (int db = 0; db < PG::NB; ++db) acc[db] = mfma<F16>(a[db], pl[u], acc[db]);
+        for (int db = 0; db < PG::NB; ++db) {
+          f4& x = acc[kLo ? PG::NB + db : db];
+          x = mfma<F16>(a[db], pl[u], x);
+        }
       }
     }
     if (wave < 4) {
@@ -847,6 +855,11 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
     } else {
       run(std::false_type{});
     }
+  }
+
+  if constexpr (kLo) {
+#pragma unroll
+    for (int db = 0; db < PG::NB; ++db) acc[db] = join_terms(acc[db], acc[PG::NB + db]);
   }
 
   // ---- normalise and store: lane (quad, r) holds dims 16 db + 4 quad + i of row r ----

@@ -166,3 +166,42 @@ def _nan_rows(L, N):
     rest = torch.ones(4, L, dtype=torch.bool)
     rest[1, 2] = rest[3, 0] = False
     assert float((out[0][rest].float() - want[0][rest].float()).abs().max()) < 2e-3
+
+
+@pytest.mark.parametrize("dtype,bits", [(F16, 4), (F16, 8), (BF16, 4), (BF16, 8)])
+@pytest.mark.parametrize("L", [1, 5, 300])
+def test_small_weights_beside_a_large_one(device, L, dtype, bits):
+    """One key (an attention sink) holds nearly all of the softmax and its
+    value is zero, so the output is the sum over keys of weight 2^-21: they
+    keep float32's precision (16-bit terms of a fixed scale would be off by
+    percents).  An output is off by its rounding (allowed twice), and by
+    scores rounded in float32: 2^-14 of the sum of the weighted |V|."""
+    Hq, Hkv, N, gs = 8, 2, 4096, 32
+    g = torch.Generator(device="cuda").manual_seed(bits + L)
+    u = torch.where(torch.rand(D, generator=g, device=device) < 0.5, 3.0, -3.0)
+    kw = torch.randn(1, Hkv, N, D, generator=g, device=device) * 0.5
+    vw = torch.randn(1, Hkv, N, D, generator=g, device=device) * 512
+    kw[:, :, 7], vw[:, :, 7] = u, 0.0
+    k, v = (kernels.quantize(x.to(dtype), gs, bits) for x in (kw, vw))
+    q = (u * 0.2 + torch.randn(1, Hq, L, D, generator=g, device=device) * 0.3).to(dtype)
+    print(f"sink L={L} {dtype} bits={bits}", flush=True)
+    out = mq.quantized_sdpa(q, k[0], v[0], k[1], v[1], k[2], v[2], bits=bits, group_size=gs)
+    kd, vd = (to.dequantize(*x, gs, bits, dtype).double().repeat_interleave(Hq // Hkv, 1) for x in (k, v))
+    assert bool((vd[:, :, 7] == 0).all())
+    p = torch.softmax(torch.matmul(q.double(), kd.transpose(2, 3).contiguous()) * D ** -0.5, -1)
+    assert 2.0 ** -24 < float(p[..., :7].median()) < 2.0 ** -18
+    want, size = torch.matmul(p, vd), torch.matmul(p, vd.abs())
+    ulp = 2.0 ** -11 if dtype == F16 else 2.0 ** -8
+    err = (out.double() - want).abs()
+    assert bool((err <= 2 * ulp * want.abs() + 2.0 ** -14 * size + 2.0 ** -24).all()), \
+        f"{float((err / size).max()):.2e} of the weighted values"
+
+
+def test_an_infinite_value_stays_infinite(device):
+    """A value past float16's range (codes of a group near it round up to
+    infinity) makes the dims that read it infinite, as float32 weights do."""
+    for L in (1, 5, 300):
+        q, k, v = _inputs(1, 4, 1, 6000, L, 8, 32, F16)
+        v[2][0, 0, 50, 1] = float("inf")  # the bias of dims 32..63
+        out = mq.quantized_sdpa(q, k[0], v[0], k[1], v[1], k[2], v[2], bits=8, group_size=32)
+        assert bool(torch.isposinf(out[..., 32:]).all()) and bool(torch.isfinite(out[..., :32]).all())
