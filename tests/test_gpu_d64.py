@@ -205,3 +205,15 @@ def test_an_infinite_value_stays_infinite(device):
         v[2][0, 0, 50, 1] = float("inf")  # the bias of dims 32..63
         out = mq.quantized_sdpa(q, k[0], v[0], k[1], v[1], k[2], v[2], bits=8, group_size=32)
         assert bool(torch.isposinf(out[..., 32:]).all()) and bool(torch.isfinite(out[..., :32]).all())
+
+
+@pytest.mark.parametrize("alone", ["keys", "values"])
+def test_biases_of_one_alone(device, alone):
+    """Several positions with the biases of the keys or of the values alone:
+    dequantize + attention's results, where they count."""
+    q, k, v = _inputs(2, 4, 2, 300, 3, 4, 32, F16)
+    k, v = (k, (v[0], v[1], None)) if alone == "keys" else ((k[0], k[1], None), v)
+    for mask in (None, "causal"):
+        out = mq.quantized_sdpa(q, k[0], v[0], k[1], v[1], k[2], v[2], mask=mask)
+        want = mq.fallback_sdpa(q, k, v, bits=4, group_size=32, scale=D ** -0.5, mask=mask)
+        assert torch.equal(out, want)
