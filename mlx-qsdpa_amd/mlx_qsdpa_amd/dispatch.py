@@ -27,6 +27,7 @@ that same dequantize + attention path at every qL.
 from __future__ import annotations
 
 import torch
+from torch.autograd import forward_ad
 
 from . import _lib, kernels
 
@@ -147,7 +148,7 @@ def quantized_sdpa(
         several = q.shape[2] > 1
         both = k_biases is not None and v_biases is not None
         if not several or q.shape[3] != 64 or (packed_k.dim() == 4 and _d64_in_kernel(
-                mask, kv_start, q.shape[0], q.shape[1], q.shape[2], packed_k.shape[2], k_biases, v_biases)):
+                q, packed_k.shape[2], mask, kv_start, k_biases, v_biases)):
             out = kernels.decode_native(q, packed_k, packed_v, k_scales, v_scales, k_biases if both else None,
                                         v_biases if both else None,
                                         scale=q.shape[3] ** -0.5 if scale is None else scale, bits=bits,
@@ -171,7 +172,7 @@ def quantized_sdpa(
         kv_start = kernels.to_device(kv_start, q.device)
 
     if D not in kernels.HEAD_DIMS or (qL > 1 and not (
-            (D != 64 or _d64_in_kernel(mask, kv_start, B, H_q, qL, N, k_biases, v_biases))
+            (D != 64 or _d64_in_kernel(q, N, mask, kv_start, k_biases, v_biases))
             and _fused_takes(q, packed_k, packed_v, k_scales, v_scales, k_biases, v_biases, scale, bits,
                              group_size))):
         return fallback_sdpa(q, (packed_k, k_scales, k_biases),    # dispatch.py:68-83
@@ -217,15 +218,17 @@ def _row_aligned(t):
 D64_FUSED_KEYS = 256
 
 
-def _d64_in_kernel(mask, kv_start, B, H_q, qL, N, k_biases, v_biases):
+def _d64_in_kernel(q, N, mask, kv_start, k_biases, v_biases):
     """Whether several positions at D = 64 run fused: enough keys, biases of
     both or of neither (one alone counts there, and not in the kernel), and
     masked as the dequantize + attention path masks them ("causal" or a bool
     mask over all keys, one start per sequence).  The path's other masks stay on
     it: additive ones (a row whose every score is the type's lowest value
     averages V there and is empty in the kernel, which scales the mask to
-    base 2), masks that broadcast over the keys."""
-    if N < D64_FUSED_KEYS or (k_biases is None) != (v_biases is None):
+    base 2), masks that broadcast over the keys.  So do calls whose queries
+    carry a gradient, which goes through its torch operations."""
+    B, H_q, qL, _ = q.shape
+    if N < D64_FUSED_KEYS or (k_biases is None) != (v_biases is None) or _differentiated(q):
         return False
     if kv_start is not None and tuple(kv_start.shape) != (B,):
         return False
@@ -235,6 +238,12 @@ def _d64_in_kernel(mask, kv_start, B, H_q, qL, N, k_biases, v_biases):
         return False
     shape = (1,) * (4 - mask.dim()) + tuple(mask.shape)
     return shape[3] == N and shape[2] in (1, qL) and shape[1] in (1, H_q) and shape[0] in (1, B)
+
+
+def _differentiated(q):
+    """Whether a gradient, of either mode, is taken through q."""
+    return (q.requires_grad and torch.is_grad_enabled()) \
+        or (forward_ad._current_level >= 0 and forward_ad.unpack_dual(q).tangent is not None)
 
 
 def _fused_takes(q, packed_k, packed_v, k_scales, v_scales, k_biases, v_biases, scale, bits,

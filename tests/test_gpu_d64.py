@@ -217,3 +217,26 @@ def test_biases_of_one_alone(device, alone):
         out = mq.quantized_sdpa(q, k[0], v[0], k[1], v[1], k[2], v[2], mask=mask)
         want = mq.fallback_sdpa(q, k, v, bits=4, group_size=32, scale=D ** -0.5, mask=mask)
         assert torch.equal(out, want)
+
+
+def test_queries_with_a_gradient(device):
+    """Several positions with a gradient of either mode through the queries:
+    dequantize + attention's torch operations."""
+    q, k, v = _inputs(2, 4, 2, 300, 3, 4, 32, F16)
+    call = lambda x: mq.quantized_sdpa(x, k[0], v[0], k[1], v[1], k[2], v[2], mask="causal")  # noqa: E731
+    path = lambda x: mq.fallback_sdpa(x, k, v, bits=4, group_size=32, scale=D ** -0.5, mask="causal")  # noqa: E731
+    plain, tangent = call(q), torch.randn_like(q)
+    grads = []
+    for f in (call, path):
+        x = q.clone().requires_grad_()
+        out = f(x)
+        out.backward(tangent)
+        grads.append(x.grad)
+        with torch.no_grad():
+            assert f(x).grad_fn is None
+    assert torch.equal(*grads) and float(grads[0].abs().max()) > 0
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(q, tangent)
+        got, want = (torch.autograd.forward_ad.unpack_dual(f(dual)) for f in (call, path))
+        assert torch.equal(got.tangent, want.tangent)
+    assert float((plain.float() - path(q).float()).abs().max()) < 2e-3

@@ -489,3 +489,24 @@ def test_a_rejected_update_leaves_the_cache_as_it_was(cpu_kernels, rng, monkeypa
     assert before == ((int(c._idx), c.offset.tolist()) if batch else c.offset)
     c.update_and_fetch(*_kv(rng, 2, 3, 5, 64))
     assert c._keys[0].shape[2] >= held + 5
+
+
+def test_routing_of_several_64_wide_positions():
+    """What leaves the dequantize + attention path at D = 64."""
+    from mlx_qsdpa_amd import dispatch
+    q, b = torch.zeros(2, 4, 3, 64), torch.zeros(1)
+
+    def fused(q=q, n=300, mask=None, start=None, kb=b, vb=b):
+        return dispatch._d64_in_kernel(q, n, mask, start, kb, vb)
+
+    assert fused() and fused(mask="causal") and fused(kb=None, vb=None) and fused(start=torch.zeros(2))
+    assert all(fused(mask=torch.ones(s, dtype=torch.bool)) for s in ((300,), (3, 300), (1, 1, 1, 300), (2, 4, 3, 300)))
+    assert not fused(kb=None) and not fused(vb=None)
+    assert not fused(mask=torch.zeros(3, 300)) and not fused(mask=torch.ones(3, 1, dtype=torch.bool))
+    assert not fused(start=torch.zeros(1))
+    g = torch.zeros(2, 4, 3, 64, requires_grad=True)
+    assert not fused(q=g)
+    with torch.no_grad():
+        assert fused(q=g)
+    with torch.autograd.forward_ad.dual_level():
+        assert fused() and not fused(q=torch.autograd.forward_ad.make_dual(q, q))
