@@ -15,8 +15,8 @@ choices:
 * Several query positions (qL > 1: speculative or chunked decoding,
   prefill) run on the fused matrix-core kernel, including mask="causal"
   (aligned to the last key), where the reference dequantizes and runs SDPA.
-  Shapes that kernel does not take (unaligned views; at D = 64 short key
-  ranges and additive masks) keep the reference's path: HIP dequantize, then
+  Shapes that kernel does not take (unaligned views; at D = 64 additive
+  masks and gradients) keep the reference's path: HIP dequantize, then
   float32 attention with torch on the GPU (dispatch.py:68-83).
 
 Head dims the library does not compile (any other multiple of 32, e.g. 32
@@ -211,24 +211,19 @@ def _row_aligned(t):
     return t.contiguous()
 
 
-# At D = 64 several query positions take the fused kernel from this many keys
-# on (a causal prompt of 1500 tokens, 32 / 8 heads: 114 us against 878 on the
-# dequantize + attention path); shorter calls are bound by their launches
-# either way.
-D64_FUSED_KEYS = 256
-
-
 def _d64_in_kernel(q, N, mask, kv_start, k_biases, v_biases):
-    """Whether several positions at D = 64 run fused: enough keys, biases of
-    both or of neither (one alone counts there, and not in the kernel), and
-    masked as the dequantize + attention path masks them ("causal" or a bool
-    mask over all keys, one start per sequence).  The path's other masks stay on
-    it: additive ones (a row whose every score is the type's lowest value
+    """Whether several positions at D = 64 run fused: biases of both or of
+    neither (one alone counts there, and not in the kernel), and masked as the
+    dequantize + attention path masks them ("causal" or a bool mask over all
+    keys, one start per sequence).  Fused they are the faster ones at every
+    size: 8 to 26 us a call against 172 to 242 on that path for 2 to 255
+    positions over 2 to 255 keys (1 to 8 sequences, 8 / 2 to 32 / 8 heads), 43
+    against 878 at 1500 of each.  The path's other masks stay on it: additive ones (a row whose every score is the type's lowest value
     averages V there and is empty in the kernel, which scales the mask to
     base 2), masks that broadcast over the keys.  So do calls whose queries
     carry a gradient, which goes through its torch operations."""
     B, H_q, qL, _ = q.shape
-    if N < D64_FUSED_KEYS or (k_biases is None) != (v_biases is None) or _differentiated(q):
+    if N < 1 or (k_biases is None) != (v_biases is None) or _differentiated(q):
         return False
     if kv_start is not None and tuple(kv_start.shape) != (B,):
         return False

@@ -219,6 +219,20 @@ def test_biases_of_one_alone(device, alone):
         assert torch.equal(out, want)
 
 
+@pytest.mark.parametrize("dtype,bits", [(F16, 4), (BF16, 8)])
+def test_several_positions_over_few_keys(device, monkeypatch, dtype, bits):
+    """The shortest calls run fused too: key ranges within one tile and just
+    past it, and positions that outnumber the keys (causal: zero rows)."""
+    monkeypatch.setattr(dispatch, "fallback_sdpa", None)
+    for B, Hq, Hkv, N, L in ((1, 4, 1, 1, 2), (2, 8, 2, 31, 31), (1, 14, 2, 33, 2), (2, 16, 1, 100, 100), (1, 8, 8, 20, 37),
+                             (3, 32, 8, 255, 255)):
+        q, k, v = _inputs(B, Hq, Hkv, N, L, bits, 32, dtype)
+        out = _check(q, k, v, bits, 32, mask="causal")
+        assert not bool(out[:, :, :max(0, L - N)].any())
+        _check(q, k, v, bits, 32, kv_start=torch.tensor([0, N // 2, N - 1][:B], device=device))
+        _check(q, k, v, bits, 32, mask=torch.rand(B, 1, L, N, device=device) < 0.5)
+
+
 def test_queries_with_a_gradient(device):
     """Several positions with a gradient of either mode through the queries:
     dequantize + attention's torch operations."""

@@ -37,7 +37,7 @@ from oracle import caches as oc
 from test_cache_invariants import CASES as WINDOW_CASES, run_window_invariants
 
 import mlx_qsdpa_amd as mq
-from mlx_qsdpa_amd import kernels
+from mlx_qsdpa_amd import dispatch, kernels
 
 pytestmark = pytest.mark.gpu
 
@@ -310,10 +310,9 @@ def test_rotating_window_invariants_on_gpu(device, kind, case):
 @pytest.mark.parametrize("layout", ["D64", "scales-2B-aligned"])
 def test_multi_query_fallback_path(device, monkeypatch, layout):
     """Shapes the fused kernel does not take for qL > 1 run the reference's
-    path (dispatch.py:68-83): HIP dequantize, float32 attention.  The fused
-    kernel is made to fail, so passing proves the fallback ran; causal, a
-    bool mask and kv_start (folded into the mask) are covered.  Layouts: D =
-    64, and K scale / bias rows only 2-byte aligned where the matrix-core
+    path (dispatch.py:68-83): HIP dequantize, float32 attention, counted
+    here.  Causal, a bool and an additive mask and kv_start (folded into the
+    mask) are covered.  Layouts: D = 64 under an additive mask, and K scale / bias rows only 2-byte aligned where the matrix-core
     kernel reads a quarter row's two groups as one 32-bit word (D = 256,
     group_size = 32)."""
     B, Hq, Hkv, N, L = 2, 8, 2, 200, 6
@@ -343,8 +342,11 @@ def test_multi_query_fallback_path(device, monkeypatch, layout):
         raise AssertionError("the fused kernel ran")
 
     monkeypatch.setattr(kernels, "decode", no_fused)
+    ran, path = [], dispatch.fallback_sdpa
+    monkeypatch.setattr(dispatch, "fallback_sdpa", lambda *a, **k: ran.append(1) or path(*a, **k))
     starts = np.array([0, 37])
-    for mask in ("causal", "bool", None):
+    # (64-wide heads: the fused kernel takes every mask but additive ones.)
+    for n, mask in enumerate(("additive",) if layout == "D64" else ("causal", "bool", "additive", None)):
         m_t = m_np = None
         if mask == "causal":
             m_t = m_np = "causal"
@@ -352,14 +354,20 @@ def test_multi_query_fallback_path(device, monkeypatch, layout):
             m_np = rng.random((B, 1, L, N)) > 0.4
             m_np[..., -1] = True
             m_t = torch.from_numpy(m_np).to(device)
+        elif mask == "additive":
+            m_np = affine.random_T(rng, (B, 1, L, N), dt)
+            m_t = from_np(m_np, T, device)
         got = mq.quantized_sdpa(dev(q), dk[0], dv[0], dk[1], dv[1], dk[2], dv[2], bits=bits, group_size=gs,
                                 mask=m_t, kv_start=torch.tensor(starts, dtype=torch.int32, device=device))
+        assert len(ran) == n + 1
         keep = np.arange(N)[None, None, None, :] >= starts[:, None, None, None]
         if mask == "causal":
             qi = np.arange(L)[:, None] + (N - L)
             full = keep & (qi >= np.arange(N)[None, :])[None, None]
         elif mask == "bool":
             full = keep & m_np
+        elif mask == "additive":
+            full = np.where(keep, m_np, -np.inf).astype(np.float32)
         else:
             full = np.broadcast_to(keep, (B, 1, L, N))
         want = attention.quantized_sdpa_reference(q, kq[0], vq[0], kq[1], vq[1], kq[2], vq[2], bits=bits,

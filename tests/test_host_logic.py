@@ -501,6 +501,7 @@ def test_routing_of_several_64_wide_positions():
 
     assert fused() and fused(mask="causal") and fused(kb=None, vb=None) and fused(start=torch.zeros(2))
     assert all(fused(mask=torch.ones(s, dtype=torch.bool)) for s in ((300,), (3, 300), (1, 1, 1, 300), (2, 4, 3, 300)))
+    assert fused(n=1) and not fused(n=0)
     assert not fused(kb=None) and not fused(vb=None)
     assert not fused(mask=torch.zeros(3, 300)) and not fused(mask=torch.ones(3, 1, dtype=torch.bool))
     assert not fused(start=torch.zeros(1))
