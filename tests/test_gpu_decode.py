@@ -658,52 +658,55 @@ def test_plan_grows_in_place_with_appends(device):
         plan.set_keys(cap + 1)
 
 
-def test_decode_argument_cache(device):
-    """kernels.decode re-launches a cached argument block for a repeated
-    tensor geometry (key count free): every cached call, over a growing key
-    count, with kv_start and on a second stream, equals the uncached call
-    bit for bit and the oracle to tolerance."""
+def test_decode_workspaces(device, monkeypatch):
+    """A thread's decode calls share one workspace per stream, grown to the
+    largest: over key counts that rise and fall, with kv_start and on a second
+    stream, every call equals the general path's on a workspace of its own bit
+    for bit and the oracle to tolerance."""
     rng = np.random.default_rng(61)
     B, Hq, Hkv, D, bits, gs, cap = 2, 16, 2, 128, 4, 64, 3000
     inp = make_inputs(rng, B, Hq, Hkv, cap, D, bits, gs)
     g = to_dev(inp, device)
     ks = torch.tensor([0, 37], dtype=torch.int32, device=device)
     side = torch.cuda.Stream(device)
+    names = ("kp", "vp", "ks", "vs", "kb", "vb")
 
-    def call(n, kv_start, cached):
-        if not cached:
-            kernels._ARGS.d = {}
-        v = [g[k][:, :, :n] for k in ("kp", "vp", "ks", "vs", "kb", "vb")]
-        return kernels.decode(g["q"], *v, scale=D ** -0.5, bits=bits, group_size=gs, kv_start=kv_start)
+    def call(n, kv_start, **kw):
+        return kernels.decode(g["q"], *(g[k][:, :, :n] for k in names), scale=D ** -0.5, bits=bits, group_size=gs,
+                              kv_start=kv_start, **kw)
 
+    kernels._ARGS.d = {}
+    sizes = []
     for kv_start in (None, ks):
         for n in (100, 2047, 2048, 3000, 64, 1):
-            print(f"argument cache n={n} kv_start={kv_start is not None}", flush=True)
-            want = call(n, kv_start, cached=False)
-            got = call(n, kv_start, cached=True)       # hit (cached by the call above)
-            nxt = call(min(n + 1, cap), kv_start, cached=True)  # hit with another key count
+            print(f"workspaces n={n} kv_start={kv_start is not None}", flush=True)
+            with monkeypatch.context() as m:
+                m.setattr(kernels, "_native_decode", lambda *a: None)
+                want = call(n, kv_start, workspace=torch.zeros(1 << 24, dtype=torch.uint8, device=device))
+            got, nxt = call(n, kv_start), call(min(n + 1, cap), kv_start)
             with torch.cuda.stream(side):
-                other = call(n, kv_start, cached=True)  # a new entry for the other stream
+                other = call(n, kv_start)
             torch.cuda.synchronize()
-            assert torch.equal(got, want), f"n={n}: cached call differs"
+            assert torch.equal(got, want), f"n={n}: shared workspace differs"
             assert torch.equal(other, want), f"n={n}: other stream differs"
-            sub = {k: (None if inp[k] is None else inp[k][:, :, :min(n + 1, cap)]) for k in inp
-                   if k in ("kp", "vp", "ks", "vs", "kb", "vb")}
-            ref_in = dict(inp, **sub)
+            held = kernels._ARGS.d
+            assert set(held) <= {(0, 0), (0, side.cuda_stream)}
+            sizes.append(held[0, 0].numel() if (0, 0) in held else 0)
+            sub = {k: (None if inp[k] is None else inp[k][:, :, :min(n + 1, cap)]) for k in names}
             mask = None
             if kv_start is not None:
                 mask = np.arange(min(n + 1, cap))[None, None, None, :] >= np.array([0, 37])[:, None, None, None]
                 if min(n + 1, cap) <= 37:
                     continue  # sequence 1 has no keys: its row is all-masked
-            assert_close(to_np(nxt), oracle_out(ref_in, mask=mask), f"n={n + 1} cached")
+            assert_close(to_np(nxt), oracle_out(dict(inp, **sub), mask=mask), f"n={n + 1}")
+    assert sizes == sorted(sizes) and 0 < sizes[-1] and len(kernels._ARGS.d) == 2
 
 
-def test_argument_cache_keys_on_alignment(device):
-    """A cached argument block is re-used only for views with the same
-    pointer alignment: the same geometry with q, or the K scales, one
-    element (2 bytes) off a 4-byte boundary takes another plan (the
-    matrix-core kernel reads them as 32-bit words), and each call still
-    matches the oracle, before and after the aligned block is cached."""
+def test_plan_follows_alignment(device):
+    """Every call is planned for its own views: the same geometry with q, or
+    the K scales, one element (2 bytes) off a 4-byte boundary takes another
+    kernel (the matrix-core one reads them as 32-bit words), and matches the
+    oracle before and after a call with aligned ones."""
     rng = np.random.default_rng(62)
     B, Hq, Hkv, N, D, bits, gs = 1, 16, 2, 4000, 256, 4, 32
     inp = make_inputs(rng, B, Hq, Hkv, N, D, bits, gs)
@@ -718,11 +721,9 @@ def test_argument_cache_keys_on_alignment(device):
         assert v.stride() == t.stride() and v.data_ptr() % 4 == 2
         return v
 
-    kernels._ARGS.d = {}
     for name in ("q", "ks"):
         for order in ("aligned first", "shifted first"):
-            print(f"alignment key: {name} {order}", flush=True)
-            kernels._ARGS.d = {}
+            print(f"alignment: {name} {order}", flush=True)
             alt = dict(g, **{name: shifted(g[name])})
             seq = (g, alt, g, alt) if order == "aligned first" else (alt, g, alt, g)
             for t in seq:

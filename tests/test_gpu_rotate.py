@@ -54,6 +54,21 @@ def test_rotate(device, B, Hq, Hkv, L, D, projected, dtype):
     assert ((got[0].double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("theta", [10000.0, 500000.0])
+@pytest.mark.parametrize("B,Hq,Hkv,L,D", [(2, 16, 4, 1, 128), (1, 3, 1, 700, 64), (3, 8, 2, 5, 256), (2, 4, 4, 9, 96),
+                                          (1, 2, 2, 3, 80)])
+def test_rotate_gives_the_bits_of_the_expression(device, B, Hq, Hkv, L, D, theta, dtype):
+    """Operation for operation the layer's torch expression on the GPU."""
+    g = torch.Generator(device="cuda").manual_seed(B + D)
+    q, k = ((torch.randn(B, L, h, D, generator=g, device="cuda") * 3).to(dtype).transpose(1, 2) for h in (Hq, Hkv))
+    for start in (torch.arange(B) * 1777 + 3, torch.full((B,), 65000)):
+        got = kernels.rotate(q, k, start, theta)
+        pos = start[:, None] + torch.arange(L)[None, :]
+        for y, x in zip(got, (q, k)):
+            assert torch.equal(y, attention._rope(x, pos, theta))
+
+
 def test_other_calls_keep_the_expression(device):
     q, k = torch.randn(2, 4, 3, 64, device="cuda").half(), torch.randn(2, 2, 3, 64, device="cuda").half()
     assert kernels.rotate(q.float(), k.float(), 0, 1e4) is None
