@@ -355,10 +355,10 @@ struct Prefill {
 // them.  Memory-latency bound; 7.6 us traced for 8 masks of 500 x 1500 bools, a
 // launch included.
 //
-// What it is worth (that chunk, 32 / 8 heads, 8-bit bf16, the call): 172 us
+// What it is worth (that chunk, 32 / 8 heads, 8-bit bf16, the call): 170 us
 // under the batch cache's mask against 202 over every tile.  What it costs: a
-// mask that leaves no tile out (all true, or holes everywhere) takes 218
-// against 201.  Calls that cannot gain go without (prefill_range_bytes).  The
+// mask that leaves no tile out (all true, or holes everywhere) takes 211
+// against 203.  Calls that cannot gain go without (prefill_range_bytes).  The
 // same look inside the prefill kernel, by each workgroup for itself, was 38 us
 // slower, a list there of the tiles with an attended key 27 us (and 42 us
 // slower for a mask with holes everywhere: an index from the LDS per tile).
@@ -384,13 +384,64 @@ __device__ __forceinline__ bool mask_word(uint32_t w) {
   }
 }
 
-// Grid (key chunks, row groups, B): the first attended key of the group's
+// Whether the sequences' last rows attend to runs of keys whose lengths differ
+// by more than an eighth of the longest (at most 64 sequences are looked at):
+// the order of the prefill's workgroups follows it (the XCDs' heads), nothing
+// else.  One wave per sequence, by one workgroup.
+template <int KIND>
+__device__ __forceinline__ bool mask_uneven(const MfmaParams& p) {
+  constexpr int ES = mask_bytes(KIND), E = 16 / ES;
+  __shared__ int s_min, s_max;
+  const int lane = threadIdx.x & 63;
+  if (threadIdx.x == 0) {
+    s_min = 0x7FFFFFFF;
+    s_max = 0;
+  }
+  __syncthreads();
+  const int n = min(p.B, 64);
+  for (int i = threadIdx.x >> 6; i < n; i += 8) {
+    const int b = static_cast<int>(static_cast<int64_t>(i) * p.B / n);
+    const uint8_t* row = static_cast<const uint8_t*>(p.mask) +
+                         (static_cast<int64_t>(b) * p.m_sb + static_cast<int64_t>(p.qL - 1) * p.m_sq) * ES;
+    int lo = 0x7FFFFFFF, hi = 0;
+    for (int k0 = lane * E; k0 < p.N && p.N >= E; k0 += 64 * E) {
+      const int k = min(k0, p.N - E);  // the last column ends with the row
+      u4 w;
+      __builtin_memcpy(&w, row + static_cast<int64_t>(k) * ES, 16);
+      if (mask_word<KIND>(w[0]) || mask_word<KIND>(w[1]) || mask_word<KIND>(w[2]) || mask_word<KIND>(w[3])) {
+        lo = min(lo, k);
+        hi = max(hi, k + E);
+      }
+    }
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      lo = min(lo, __shfl_xor(lo, o));
+      hi = max(hi, __shfl_xor(hi, o));
+    }
+    if (lane == 0) {
+      atomicMin(&s_min, max(hi - lo, 0));
+      atomicMax(&s_max, max(hi - lo, 0));
+    }
+  }
+  __syncthreads();
+  return s_max - s_min > s_max / 8;
+}
+
+// Grid (key chunks, row groups + 1, B): the first attended key of the group's
 // positions in the chunk and one past the last, in columns of 16 bytes of
-// mask, to ranges[(b * groups + group) * chunks + chunk] (0, 0: none).  A
-// thread takes a column down its share of the rows, eight loads in flight.
+// mask, to ranges[(b * groups + group) * chunks + chunk] (0, 0: none); past
+// those, by one workgroup of the last group, mask_uneven.  A thread takes a
+// column down its share of the rows, eight loads in flight.
 // (Rows start at any byte: the loads are unaligned ones.)
 template <int KIND>
 __global__ __launch_bounds__(512) void mask_range_kernel(MfmaParams p, int chunk) {
+  const int groups = gridDim.y - 1;
+  if (blockIdx.y == static_cast<unsigned>(groups)) {
+    if (blockIdx.x != 0 || blockIdx.z != 0) return;
+    const bool uneven = p.B > 1 && p.m_sb != 0 && mask_uneven<KIND>(p);
+    if (threadIdx.x == 0) p.ranges[static_cast<int64_t>(p.B) * groups * gridDim.x] = int2{uneven ? 1 : 0, 0};
+    return;
+  }
   constexpr int ES = mask_bytes(KIND), E = 16 / ES;  // keys per column
   constexpr int U = 8;
   __shared__ int s_lo, s_hi;
@@ -438,7 +489,7 @@ __global__ __launch_bounds__(512) void mask_range_kernel(MfmaParams p, int chunk
   }
   __syncthreads();
   if (tid == 0) {
-    const int64_t at = (static_cast<int64_t>(blockIdx.z) * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x;
+    const int64_t at = (static_cast<int64_t>(blockIdx.z) * groups + blockIdx.y) * gridDim.x + blockIdx.x;
     p.ranges[at] = s_hi > 0 ? int2{s_lo, min(s_hi, p.N)} : int2{0, 0};
   }
 }
@@ -473,17 +524,19 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
   // holds only long groups.  A prompt of 3000 tokens (32 / 8 heads, 4-bit; 752
   // workgroups), with its cache update: 142.6 us against 156.5 with the
   // shortest groups first.  Where the sequences' key ranges may differ (a
-  // start each, or a mask's ranges), an XCD takes every eighth head, so that
+  // start each) or do (mask_uneven), an XCD takes every eighth head, so that
   // it does not hold one sequence alone: 8 sequences of 500 x 1500 (32 / 8
-  // heads, 8-bit bf16), kernel alone, under the batch cache's mask 182 us
-  // against 221 in runs (227 without the ranges); a mask with random holes
-  // everywhere 229 against 226 (221).  A mask without ranges keeps the runs:
-  // 2 sequences of 512 x 2048 in one round of 256 workgroups 64.1 against 66.0.
+  // heads, 8-bit bf16) under the batch cache's mask 182 us traced against 221
+  // in runs.  Others keep the runs, in which an XCD reads one sequence's mask:
+  // the call under one with random holes everywhere 211 us against 218, 2
+  // sequences of 512 x 2048 in one round of workgroups 64.1 against 66.0.
   const int total = gridDim.x;
   const int heads = p.Hkv * p.B;
   const int S = p.num_splits;
   const bool ranged = MASK && p.ranges;
-  const bool uneven = p.B > 1 && ((ranged && p.m_sb != 0) || p.kv_start);
+  bool uneven = p.B > 1 && p.kv_start;
+  if (ranged && p.B > 1 && !uneven)
+    uneven = p.ranges[static_cast<int64_t>(p.B) * groups_per_head * p.range_chunks].x != 0;
   int w = blockIdx.x, split = 0, grp, head;
   if ((p.causal || ranged || uneven) && S == 1 && heads % 8 != 0) {
     head = w % heads;
@@ -938,7 +991,7 @@ void launch_mask_range(const MfmaParams& p, int groups, hipStream_t stream) {
                                : p.mask_kind == QSDPA_F16 ? mask_range_kernel<QSDPA_F16>
                                : p.mask_kind == QSDPA_BF16 ? mask_range_kernel<QSDPA_BF16>
                                                            : mask_range_kernel<QSDPA_F32>;
-  hipLaunchKernelGGL(k, dim3(p.range_chunks, groups, p.B), dim3(512), 0, stream, p, chunk);
+  hipLaunchKernelGGL(k, dim3(p.range_chunks, groups + 1, p.B), dim3(512), 0, stream, p, chunk);
 }
 
 template <typename Tag, int D, int BITS, bool MASK>
@@ -1059,10 +1112,10 @@ int prefill_num_splits(const qsdpa_decode_args* a, int cus) {
 int64_t prefill_range_bytes(const qsdpa_decode_args* a, int splits, int cus) {
   if (!a->mask.ptr || a->mask.stride_n != 1 || a->mask.stride_h != 0) return 0;
   const int64_t groups = (static_cast<int64_t>(a->H_q / a->H_kv) * a->q_len + kPGroupRows - 1) / kPGroupRows;
-  if (groups > 65535 || a->B > 65535) return 0;
+  if (groups > 65534 || a->B > 65535) return 0;
   if (splits > 1 || groups * a->H_kv * a->B <= cus) return 0;
   const int64_t chunks = (a->N + range_chunk(a->N) - 1) / range_chunk(a->N);
-  return (groups * a->B * chunks * 8 + 255) / 256 * 256;
+  return ((groups * a->B * chunks + 1) * 8 + 255) / 256 * 256;
 }
 
 int launch_prefill_mfma(const qsdpa_decode_args* a, int splits, float* part_acc, float* part_ml, void* ranges,
