@@ -351,7 +351,7 @@ class QuantizedSDPACache:
         """Quantize keys/values (B, H_kv, S, D) and append them (cache.py:163-197)."""
         _append(self, keys, values, self.offset)
         self.offset += keys.shape[2]
-        return _sl(self._keys, 0, self.offset), _sl(self._values, 0, self.offset)
+        return kernels.columns(self._keys, self.offset), kernels.columns(self._values, self.offset)
 
 
 class BatchQuantizedSDPACache:
@@ -410,7 +410,7 @@ class BatchQuantizedSDPACache:
         _append(self, keys, values, self._idx)
         self.offset = self.offset + S
         self._idx += S
-        return _sl(self._keys, 0, self._idx), _sl(self._values, 0, self._idx)
+        return kernels.columns(self._keys, self._idx), kernels.columns(self._values, self._idx)
 
     def prepare(self, *, left_padding=None, lengths=None, right_padding=None):
         """cache.py:324-335."""

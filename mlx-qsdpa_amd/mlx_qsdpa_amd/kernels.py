@@ -140,7 +140,7 @@ def quantize_kv_into(keys: torch.Tensor, values: torch.Tensor, kdst: tuple, vdst
                      bits: int, group_size: int) -> None:
     """quantize_into for the keys and the values of one cache update, in one launch."""
     if keys.is_cuda:
-        rc = _host().quantize_kv(keys, values, kdst, vdst, t0, bits, group_size, _stream(keys))
+        rc = (_HOST or _host()).quantize_kv(keys, values, kdst, vdst, t0, bits, group_size, _stream(keys))
         if rc is not None:
             _lib.check(rc)
             return
@@ -226,7 +226,8 @@ def requant_window(old: tuple, new: tuple, dst: tuple, n_old: int, keep: int, ro
 
 def columns(buffers: tuple, n: int) -> tuple:
     """The first n columns (dim 2) of each of a cache's (B, H, N, W) tensors."""
-    out = _host().columns(buffers, n) if buffers[0].is_cuda else None
+    host = _HOST or (_host() if buffers[0].is_cuda else None)
+    out = None if host is None else host.columns(buffers, n)
     return tuple(t[:, :, :n, :] for t in buffers) if out is None else out
 
 
@@ -237,7 +238,7 @@ def grown(keys, values, old, prev, cols, bits, group_size):
     write).  None for tensors it does not take."""
     if not keys.is_cuda:
         return None
-    out = _host().grown(keys, values, old, prev, cols, bits, group_size, _stream(keys))
+    out = (_HOST or _host()).grown(keys, values, old, prev, cols, bits, group_size, _stream(keys))
     if type(out) is int:
         _lib.check(out)
     return out
@@ -250,7 +251,7 @@ def rotate(q, k, start, theta):
     gradient or a trace goes through q or k."""
     if not q.is_cuda or torch.jit.is_tracing() or torch.compiler.is_compiling():
         return None
-    out = _host().rotate(q, k, start, theta, _stream(q))
+    out = (_HOST or _host()).rotate(q, k, start, theta, _stream(q))
     if type(out) is int:
         _lib.check(out)
     return out
@@ -266,7 +267,7 @@ def causal_mask(N, start, pad, window, device):
     device = torch.device(device)
     if device.index is None:
         device = torch.device("cuda", torch.cuda.current_device())
-    out = _host().causal_mask(N, start, pad, window, device.index, torch.cuda.current_stream(device).cuda_stream)
+    out = (_HOST or _host()).causal_mask(N, start, pad, window, device.index, torch.cuda.current_stream(device).cuda_stream)
     if type(out) is int:
         _lib.check(out)
     return out
@@ -551,7 +552,7 @@ def _native_decode(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start,
     code, or None where that does not take the tensors."""
     stream = _stream(q)
     ws = _workspace(q.device, stream, 0)
-    fn = _host().decode
+    fn = (_HOST or _host()).decode
     out = fn(q, pk, pv, ks, vs, kb, vb, scale, bits, group_size, kv_start, num_splits, causal, ws, stream, mask)
     if type(out) is int and out > 0:
         ws = _workspace(q.device, stream, out)

@@ -443,6 +443,7 @@ def test_growth_rejects_other_shapes(cpu_kernels, rng):
 def test_caches_on_the_cpu_need_no_library(cpu_kernels, rng, monkeypatch):
     """Slices of CPU buffers (state, trim, what an update returns) are torch's
     alone: no built library."""
+    monkeypatch.setattr(pc.kernels, "_HOST", None)
     monkeypatch.setattr(pc.kernels, "_host", None)
     for c in (pc.QuantizedSDPACache(bits=4, group_size=32), pc.BatchQuantizedSDPACache([0, 0], bits=4, group_size=32)):
         k, v = _kv(rng, 2, 3, 300, 64)
