@@ -568,9 +568,9 @@ void launch_bits(const MfmaParams& p, int bits, int gs, hipStream_t stream, cons
 
 // D = 64 against the VALU kernel (decode_valu.hip), which takes only its
 // unaligned views now, wall us per call: B = 8, 32 / 8 heads over 8192 keys,
-// 4-bit f16 16.6 against 35.4, 8-bit bf16 19.2 against 42.2; B = 1 over 4096 /
-// 32768 keys 9.8 / 13.2 against 14.4 / 24.1; 16 left-padded sequences of
-// 2192 to 8192 keys (stream-K) 29.0 against 61.6.  It is VALU-bound: a tile
+// 4-bit f16 18.0 against 35.4, 8-bit bf16 19.1 against 42.2; B = 1 over 4096 /
+// 32768 keys 10.1 / 13.8 against 14.4 / 24.1; 16 left-padded sequences of
+// 2192 to 8192 keys (stream-K) 26.4 against 61.6.  It is VALU-bound: a tile
 // holds half the bytes of a D = 128 one under the same softmax.
 //
 // The MFMA path covers D in {64, 128, 256} for any GQA factor (heads padded to

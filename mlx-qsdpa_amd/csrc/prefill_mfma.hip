@@ -1045,14 +1045,15 @@ bool prefill_supports(const qsdpa_decode_args* a) {
   // heads at q_len = 4 over 128K 58-59 against 73-75 us.
   if (a->D == 256 && static_cast<int64_t>(a->B) * a->H_q * a->q_len * a->N < (int64_t(1) << 24))
     return false;
-  // D = 64 from 5 * 2^20 pairs on.  Wall us per call, the decode kernel
-  // against this one: one sequence of 32 / 8 heads, q_len = 33 over 4096 /
-  // 8192 / 16384 keys 15.6 / 21.6 / 35.0 against 16.2 / 20.3 / 27.6 (4.3 /
-  // 8.7 / 17 million pairs), q_len = 100 over 1024 (3.3 million) 10.5 against
-  // 14.3, q_len = 300 over 600 (5.8 million) 19.9 against 19.2, 200 over 2048
-  // (13 million) 26.5 against 19.2; 8 / 2 heads, q_len = 100 over 4096 (3.3
-  // million) 13.1 against 15.7.  Prompts of 1500 / 3000 tokens 98.6 / 252
-  // against 36.4 / 99.2.
+  // D = 64 from 5 * 2^20 pairs on.  Wall us per causal call (4-bit float16),
+  // the decode kernel against this one: one sequence of 32 / 8 heads, q_len =
+  // 33 over 4096 / 8192 / 16384 keys 15.4 / 21.2 / 35.1 against 17.9 / 22.0 /
+  // 29.3 (4.3 / 8.7 / 17 million pairs; 8-bit bfloat16 16.7 / 25.1 / 41.0
+  // against 18.8 / 23.2 / 31.1), q_len = 100 over 1024 (3.3 million) 11.0
+  // against 15.4, q_len = 300 over 600 (5.8 million) 20.7 against 20.9, 200
+  // over 2048 (13 million) 27.0 against 22.0; 8 / 2 heads, q_len = 100 over
+  // 4096 (3.3 million) 13.6 against 16.7.  Prompts of 1500 / 3000 tokens 93.9 /
+  // 253 against 35.2 / 102.3.
   if (a->D == 64 && static_cast<int64_t>(a->B) * a->H_q * a->q_len * a->N < (int64_t(5) << 20)) return false;
   // One row group per kv head at D = 256 goes to the 32-row decode kernel
   // where that takes the call (4-bit codes, no mask tensor, ...): C3's heads

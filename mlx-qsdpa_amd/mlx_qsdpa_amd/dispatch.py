@@ -217,7 +217,7 @@ def _d64_in_kernel(q, N, mask, kv_start, k_biases, v_biases):
     dequantize + attention path masks them ("causal" or a bool mask over all
     keys, one start per sequence).  Fused they are the faster ones at every
     size: 8 to 26 us a call against 172 to 242 on that path for 2 to 255
-    positions over 2 to 255 keys (1 to 8 sequences, 8 / 2 to 32 / 8 heads), 43
+    positions over 2 to 255 keys (1 to 8 sequences, 8 / 2 to 32 / 8 heads), 44
     against 878 at 1500 of each.  The path's other masks stay on it: additive ones (a row whose every score is the type's lowest value
     averages V there and is empty in the kernel, which scales the mask to
     base 2), masks that broadcast over the keys.  So do calls whose queries
