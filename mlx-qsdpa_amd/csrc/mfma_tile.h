@@ -426,10 +426,13 @@ struct Kernel {
     if constexpr (Tag::kId == QSDPA_BF16 || kLo) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const float x = pr[2 * i] - unpack_T2_lo<Tag>(pb[i]), y = pr[2 * i + 1] - unpack_T2_hi<Tag>(pb[i]);
-        pb_lo[i] = kLo ? pack_T2<Tag>(x * kLoScale, y * kLoScale) : pack_T2<Tag>(x, y);
-        if constexpr (G::Wide && !kLo)
-          pb_lo2[i] = pack_T2<Tag>(x - unpack_T2_lo<Tag>(pb_lo[i]), y - unpack_T2_hi<Tag>(pb_lo[i]));
+        if constexpr (kLo) {
+          pb_lo[i] = lo_terms(pb[i], pr[2 * i], pr[2 * i + 1]);
+        } else {
+          const float x = pr[2 * i] - unpack_T2_lo<Tag>(pb[i]), y = pr[2 * i + 1] - unpack_T2_hi<Tag>(pb[i]);
+          pb_lo[i] = pack_T2<Tag>(x, y);
+          if constexpr (G::Wide) pb_lo2[i] = pack_T2<Tag>(x - unpack_T2_lo<Tag>(pb_lo[i]), y - unpack_T2_hi<Tag>(pb_lo[i]));
+        }
       }
     }
 

@@ -772,10 +772,10 @@ __global__ __launch_bounds__(kPThreads) void prefill_mfma_kernel(MfmaParams p, i
       for (int i = 0; i < 4; ++i) {
         const int e = 4 * (2 * u + (i >> 1)) + 2 * (i & 1);
         pb[u][i] = pack_T2<F16>(pr[e], pr[e + 1]);
-        if constexpr (kTwo) {
-          const float x = pr[e] - unpack_T2_lo<F16>(pb[u][i]), y = pr[e + 1] - unpack_T2_hi<F16>(pb[u][i]);
-          pl[u][i] = kLo ? pack_T2<F16>(x * kLoScale, y * kLoScale) : pack_T2<F16>(x, y);
-        }
+        if constexpr (kLo)
+          pl[u][i] = lo_terms(pb[u][i], pr[e], pr[e + 1]);
+        else if constexpr (kTwo)
+          pl[u][i] = pack_T2<F16>(pr[e] - unpack_T2_lo<F16>(pb[u][i]), pr[e + 1] - unpack_T2_hi<F16>(pb[u][i]));
       }
     // ---- out^T += V^T P^T (two terms: the hi terms of all dim blocks, then the lo terms) ----
     const uint8_t* vt = cur + PG::KBytes;
