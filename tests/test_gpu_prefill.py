@@ -406,7 +406,7 @@ def _block_mask(B, L, N, seed):
 @pytest.mark.parametrize("D,bits,gs,dtype", [(128, 4, 64, torch.float16), (128, 8, 128, torch.bfloat16),
                                              (256, 4, 32, torch.float16), (256, 8, 64, torch.bfloat16),
                                              (64, 4, 32, torch.float16), (64, 8, 64, torch.bfloat16)])
-@pytest.mark.parametrize("B,Hq,Hkv,N,L", [(2, 32, 8, 1001, 333), (1, 16, 2, 4099, 130)], ids=["rounds", "splits"])
+@pytest.mark.parametrize("B,Hq,Hkv,N,L", [(3, 32, 8, 1001, 333), (1, 16, 2, 4099, 130)], ids=["rounds", "splits"])
 def test_prefill_skips_masked_tiles(device, D, bits, gs, dtype, B, Hq, Hkv, N, L):
     """Masks that rule out whole tiles at either end of a row group's keys:
     bool and additive, odd row lengths, one mask row for all positions,
@@ -418,7 +418,7 @@ def test_prefill_skips_masked_tiles(device, D, bits, gs, dtype, B, Hq, Hkv, N, L
     keep = _block_mask(B, L, N, seed=L).to(device)
     print(f"prefill block mask D={D} {dtype} N={N} L={L}", flush=True)
     _check(q, kq, vq, bits, gs, "bool", mask=keep)
-    ks = torch.tensor([77, 400][:B], dtype=torch.int32, device=device)
+    ks = torch.tensor([77, 400, 0][:B], dtype=torch.int32, device=device)
     _check(q, kq, vq, bits, gs, "bool, start, causal", mask=keep, kv_start=ks, causal=True)
     for t in (dtype, torch.float32):
         add = torch.where(keep, 0.0, float("-inf")).to(t)
@@ -433,7 +433,8 @@ def test_prefill_skips_masked_tiles(device, D, bits, gs, dtype, B, Hq, Hkv, N, L
 
 @pytest.mark.parametrize("D,bits,gs,dtype", [(128, 4, 64, torch.float16), (128, 8, 128, torch.bfloat16),
                                              (256, 4, 32, torch.float16), (64, 8, 64, torch.bfloat16)])
-@pytest.mark.parametrize("B,Hq,Hkv,N,L", [(3, 32, 8, 1001, 333), (1, 16, 2, 4099, 130)], ids=["rounds", "splits"])
+@pytest.mark.parametrize("B,Hq,Hkv,N,L", [(3, 32, 8, 1001, 333), (1, 16, 2, 4099, 130), (70, 8, 2, 200, 64)],
+                         ids=["rounds", "splits", "many"])
 def test_prefill_mask_shared_by_the_heads_gives_the_bits_of_one_each(device, D, bits, gs, dtype, B, Hq, Hkv, N, L):
     """A mask of one row set for all heads leaves out tiles, one per head does
     not: the outputs are the same bits, in one pass and with key splits (whose
@@ -444,7 +445,7 @@ def test_prefill_mask_shared_by_the_heads_gives_the_bits_of_one_each(device, D, 
     keep = _block_mask(B, L, N, seed=L + 1).to(device)
     print(f"prefill shared mask D={D} {dtype} N={N} L={L}", flush=True)
     args = (q, kq[0], vq[0], kq[1], vq[1], kq[2], vq[2])
-    start = torch.tensor([77, 400, 0][:B], dtype=torch.int32, device=device)
+    start = torch.tensor(([77, 400, 0] * B)[:B], dtype=torch.int32, device=device)
     add = torch.where(keep, 0.0, float("-inf")).to(dtype)
     add[..., 100:140] += 2.0
     for mask, kw in ((keep, {}), (keep, dict(causal=True, kv_start=start)), (add, {}), (add.float(), {}),
