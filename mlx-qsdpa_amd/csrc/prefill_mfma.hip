@@ -352,7 +352,7 @@ struct Prefill {
 // mask once, and a row group then runs from the tile of its first attended
 // key to that of its last.  Only masks whose keys are adjacent and whose rows
 // are shared by the heads: one pass over one head's mask then serves all of
-// them.  Memory-latency bound; 7.6 us traced for 8 masks of 500 x 1500 bools, a
+// them.  Memory-latency bound; 9 us traced for 8 masks of 500 x 1500 bools, a
 // launch included.
 //
 // What it is worth (that chunk, 32 / 8 heads, 8-bit bf16, the call): 170 us
